@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "conv.hpp"
+#include "igemm_split.hpp"
 #include "kernels.hpp"
 
 namespace spk::kern {
@@ -100,55 +101,6 @@ void conv_plan_free(void *p) {
 
 // ------------------------------------------------------- implicit GEMM kernel
 
-// gfx9 buffer resource word 3 (raw, untyped loads); loads whose offset is at
-// or beyond num_records return 0.
-constexpr int kBufferWord3 = 0x00020000;
-// byte offset that is out of range for every tensor (they are < 2 GiB), and
-// still does not wrap when a valid offset is added to it
-constexpr int kOobOffset = 0x7fff0000;
-
-struct IgemmArgs {
-    const float *__restrict__ x;     // B-operand source: NCHW input, zero-padded when the conv pads
-    const float *__restrict__ wp;    // [m_tiles][k_tiles] BM x BK tiles in MFMA fragment order
-    const int *__restrict__ koff;    // [Kpad + 2*BK] byte offset of k = (c, kh, kw) in x, kOobOffset past K
-    const float *__restrict__ bias;  // [M] or null
-    const float *__restrict__ res;   // like y, or null
-    float *__restrict__ y;
-    float *__restrict__ ws;          // split-K partials [splitk][M][ws_ld], column n at n - ws_n0
-    int ws_n0, ws_ld;                // first column with partials, columns per partial row
-    int dp_tiles, rem_split;         // hybrid: whole tiles first; rem_split slices per split tile
-    int x_bytes;                     // extent of x for the bounds-checked loads
-    int y_bytes;                     // extent of y (and of the residual)
-    int ws_bytes;                    // extent of the split-K partials
-    int Wp;                          // row pitch of x (padded width)
-    int M, OW, OHW, Ntot;
-    int sh, sw;
-    int x_img_stride;                // elements between images in x
-    int y_img_stride;                // elements between images in y and the residual
-    int y_cstride;                   // elements between channels in y (OHW unless y is a view)
-    int m_tiles, k_tiles, kt_per_split;
-    int act;
-    float alpha;
-    // handoff: also store the output into the consuming conv's zero-padded
-    // input (NCHW, Hp x Wp planes); y may then be null (no other reader)
-    float *__restrict__ yp;
-    int yp_bytes, yp_Wp, yp_pt, yp_pl, yp_plane;
-    int yp_m0, yp_C;  // the handed-off channels: m0 .. m0 + C - 1 of y, the target's channels 0 .. C - 1
-    // skinny kernel: k = tap * sk_C + c (a tap's channels consecutive);
-    // channel c of a tap is c * sk_cstride elements past channel 0, tap
-    // (kh, kw) = (tap / sk_KW, tap % sk_KW) kh * sk_tap_h + kw * sk_tap_w
-    // elements past tap 0
-    int sk_C, sk_cstride, sk_KW, sk_tap_h, sk_tap_w;
-    // implicit padding (kModeChk): per-k tap table ((kh*dh) << 16 | kw*dw,
-    // 0x7fff7fff past K), the unpadded input's extent and the padding
-    const int *__restrict__ ktap;
-    int chk_H, chk_W, chk_ph, chk_pw;
-    int th_steps;  // thin kernel: K / 4 MFMA steps (k' = tap * sk_C + c)
-    // row-window kernel: the input window's geometry (GatherGeom's win_*)
-    int win_KH, win_len, win_shift, win_owb, win_OH, win_dw;
-};
-
-
 // Implicit GEMM: one BM x BN output tile per 256-thread workgroup
 // (blockIdx.x), the k range optionally split over blockIdx.y (split-K
 // partials are summed by splitk_epilogue).
@@ -165,7 +117,6 @@ struct IgemmArgs {
 // each element is bounds-checked: tap table entry (kh*dh, kw*dw) of k against
 // the lane's column base (oh*sh - ph, ow*sw - pw); taps outside the input
 // load 0, so a padded conv needs no zero-padded copy of its input.
-constexpr int kModePlain = 0, kModeKvec = 1, kModeChk = 2;
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int MODE = kModePlain>
 __global__ void __launch_bounds__(256) conv_igemm_f32(IgemmArgs a) {
@@ -229,7 +180,6 @@ __global__ void __launch_bounds__(256) conv_igemm_f32(IgemmArgs a) {
         const_cast<float *>(a.x), static_cast<short>(0), a.x_bytes, kBufferWord3);
     const int row = lane & 31;
     const int khalf = 4 * (lane >> 5);
-    const int rsub = 4 * (lane >> 5);
 
     {
         int col = kOobOffset;
@@ -376,123 +326,7 @@ __global__ void __launch_bounds__(256) conv_igemm_f32(IgemmArgs a) {
 #undef IGEMM_LOAD_B
 #undef IGEMM_STORE_B
 
-        // 32x32 accumulator layout: lane holds column (lane & 31) and rows
-        // 8*(r/4) + 4*(lane/32) + (r%4) for r = 0..15.  Output offsets are
-        // 32-bit (tensors < 2 GiB); rows past M and columns past N get an
-        // out-of-range offset, so the buffer stores drop them.
-        int obase[TN];  // byte offset of (row 0, this lane's column) in y / res / ws
-        int mrow[TM];   // first row of this lane in block i
-#pragma unroll
-        for (int i = 0; i < TM; i++) mrow[i] = mt * BM + (wm * TM + i) * 32 + rsub;
-        if (part) {
-            // split-K partials: ws[slice][m][n - ws_n0], rows of ws_ld columns
-            const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-                a.ws, static_cast<short>(0), a.ws_bytes, kBufferWord3);
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int n = nt * BN + (wn * TN + j) * 32 + row;
-                obase[j] = n < a.Ntot ? (slice * a.M * a.ws_ld + n - a.ws_n0) * 4 : kOobOffset;
-            }
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
-                        const int off = m < a.M ? obase[j] + m * a.ws_ld * 4 : kOobOffset;
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r]), wrs, off, 0, 0);
-                    }
-            return;  // splitk_epilogue sums the partials
-        }
-        {
-            const int ohw4 = a.OHW * 4;      // the residual's channel stride (natural layout)
-            const int ycs4 = a.y_cstride * 4;  // y's
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int n = nt * BN + (wn * TN + j) * 32 + row;
-                const int img = n / a.OHW;
-                const int sp = n - img * a.OHW;
-                obase[j] = n < a.Ntot ? (img * a.y_img_stride + sp) * 4 : kOobOffset;
-            }
-            float *const any = a.y ? a.y : a.yp;
-            const __amdgpu_buffer_rsrc_t yrs =
-                __builtin_amdgcn_make_buffer_rsrc(any, static_cast<short>(0), a.y ? a.y_bytes : 0, kBufferWord3);
-            const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
-                a.yp ? a.yp : any, static_cast<short>(0), a.yp ? a.yp_bytes : 0, kBufferWord3);
-            const __amdgpu_buffer_rsrc_t rrs = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(a.res ? a.res : any), static_cast<short>(0), a.res ? a.y_bytes : 0, kBufferWord3);
-            const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float *>(a.bias ? a.bias : any), static_cast<short>(0), a.bias ? a.M * 4 : 0, kBufferWord3);
-            // handoff target: this lane's pixel in the padded planes
-            int pbase[TN];
-            const int plane4 = a.yp_plane * 4;
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int n = nt * BN + (wn * TN + j) * 32 + row;
-                const int img = n / a.OHW;
-                const int sp = n - img * a.OHW;
-                const int oh = sp / a.OW;
-                const int ow = sp - oh * a.OW;
-                pbase[j] = n < a.Ntot ? (img * a.yp_C * a.yp_plane + (oh + a.yp_pt) * a.yp_Wp + ow + a.yp_pl) * 4
-                                      : kOobOffset;
-            }
-            // one 32x32 block at a time: its 16 bias and 16 residual loads are
-            // all in flight before the first use
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-#pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    floatx16 v = acc[i][j];
-                    if (a.alpha != 1.0f) v *= a.alpha;
-                    if (a.bias) {
-                        floatx16 bv;
-#pragma unroll
-                        for (int r = 0; r < 16; r++)
-                            bv[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                                  brs, (mrow[i] + 8 * (r >> 2) + (r & 3)) * 4, 0, 0));
-                        v += bv;
-                    }
-                    if (a.res) {
-                        floatx16 rv;
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
-                            rv[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                                  rrs, m < a.M ? obase[j] + m * ohw4 : kOobOffset, 0, 0));
-                        }
-                        v += rv;
-                    }
-                    if (a.act == 1) {
-#pragma unroll
-                        for (int r = 0; r < 16; r++) v[r] = v[r] > 0.0f ? v[r] : 0.0f;
-                    } else if (a.act == 2) {
-#pragma unroll
-                        for (int r = 0; r < 16; r++) v[r] = apply_act(v[r], 2);
-                    }
-                    if (a.yp) {
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const unsigned mc = static_cast<unsigned>(mrow[i] + 8 * (r >> 2) + (r & 3) - a.yp_m0);
-                            __builtin_amdgcn_raw_buffer_store_b32(
-                                __float_as_uint(v[r]), prs,
-                                mc < static_cast<unsigned>(a.yp_C) ? pbase[j] + static_cast<int>(mc) * plane4 : kOobOffset,
-                                0, 0);
-                        }
-                    }
-                    if (a.y) {
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
-                            // __float_as_uint takes the element by value (a bit
-                            // cast applied to a vector element reads element 0)
-                            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), yrs,
-                                                                  m < a.M ? obase[j] + m * ycs4 : kOobOffset, 0, 0);
-                        }
-                    }
-                }
-            }
-        }
+        igemm_epilogue<BM, BN, 32, TM, TN>(a, acc, mt, nt, wm, wn, lane, part, slice);
     }
 }
 
@@ -1340,6 +1174,7 @@ struct TileCfg {
     // with skinny_waves: conv_window_f32 instead (the skinny kernel's sums,
     // the input window in LDS; convolutions only)
     bool window = false;
+    int split_threads = 0;  // > 0: conv_split_f32 (bf16 parts of the operands) with this many threads
 };
 
 #define CFGW(BM, BN, BK, WM, WN, EFF)                                                                        \
@@ -1390,6 +1225,14 @@ const TileCfg kCfgs[] = {
     // the four waves stacked along M (each 32 rows by the whole tile
     // width): every weight fragment is loaded by one wave only
     CFGWL(128, 64, 16, 4, 1, 0.95), CFGWL(128, 64, 32, 4, 1, 0.95),
+    // bf16 parts (conv_split.hip), the tuner's choice wherever the layer is
+    // large enough for the fp32 MFMA rate to bound it
+#define CFGS(BM, BN, BK, WM, WN, WPE, EFF)                                                              \
+    {BM, BN, BK, #BM "x" #BN "x" #BK, conv_split_f32<BM, BN, BK, WM, WN, WPE, kModePlain>,              \
+     conv_split_f32<BM, BN, BK, WM, WN, WPE, kModeKvec>,                                                \
+     conv_split_f32<BM, BN, BK, WM, WN, WPE, kModeChk>, EFF, 0, 0, false, 64 * WM * WN},
+    SPK_SPLIT_TILES(CFGS)
+#undef CFGS
 };
 #undef CFG
 #undef CFGW
@@ -1397,7 +1240,12 @@ const TileCfg kCfgs[] = {
 constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
 
 // threads per workgroup of configuration c
-int cfg_threads(int c) { return kCfgs[c].skinny_waves > 0 ? 64 * kCfgs[c].skinny_waves : 256; }
+int cfg_threads(int c) {
+    return kCfgs[c].skinny_waves > 0 ? 64 * kCfgs[c].skinny_waves : kCfgs[c].split_threads > 0 ? kCfgs[c].split_threads : 256;
+}
+
+// bytes a weight takes packed for configuration c
+int weight_bytes(int c) { return kCfgs[c].split_threads > 0 ? 6 : 4; }
 
 // The row-window kernel of W waves for k_tiles 64-k chunks and KH (1 or 3)
 // window rows per channel: a ring of weight chunks no deeper than the
@@ -1565,9 +1413,10 @@ std::string numerics_class(int c, const TileCounts &tc) {
     const TileCfg &t = kCfgs[c];
     if (t.skinny_waves > 0) return "skinny" + std::to_string(t.skinny_waves);
     if (t.thin_mb > 0) return "thin" + std::to_string(c);
-    if (tc.splitk <= 1) return "igemm";
+    const std::string parts = t.split_threads > 0 ? "parts" : "";
+    if (tc.splitk <= 1) return parts + "igemm";
     const std::string cut = "/" + std::to_string(tc.kt_per_split * t.BK);
-    return tc.dp_tiles > 0 ? "hybrid" + std::to_string(tc.ws_n0) + cut : "splitk" + cut;
+    return parts + (tc.dp_tiles > 0 ? "hybrid" + std::to_string(tc.ws_n0) + cut : "splitk" + cut);
 }
 
 const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
@@ -1609,9 +1458,9 @@ bool cfg_fits(int c, const GatherSpec &gs) {
 
 std::vector<int> build_koff(const GatherSpec &gs, int BK) {
     const int kpad = (gs.K + BK - 1) / BK * BK;
-    // two extra tiles of out-of-range entries: the pipeline prefetches up to
-    // two tiles past the last one
-    std::vector<int> koff(static_cast<size_t>(kpad + 2 * BK), kOobOffset);
+    // three extra tiles of out-of-range entries: the pipelines read up to
+    // three tiles past the last one
+    std::vector<int> koff(static_cast<size_t>(kpad + 3 * BK), kOobOffset);
     for (int k = 0; k < gs.K; k++) koff[k] = gs.koff(k);
     return koff;
 }
@@ -1748,7 +1597,7 @@ static int launch_igemm(hipStream_t st, int cfg, const TileCounts &tc, const Con
     a.chk_pw = gg.chk_pw;
     // 16-byte B loads need a 16-byte aligned source (a caller-bound input may not be)
     const bool kvec = gg.kvec && (reinterpret_cast<uintptr_t>(xs) & 15) == 0;
-    (kvec ? t.kernel_kvec : gg.chk ? t.kernel_chk : t.kernel)<<<grid, dim3(256), 0, st>>>(a);
+    (kvec ? t.kernel_kvec : gg.chk ? t.kernel_chk : t.kernel)<<<grid, dim3(cfg_threads(cfg)), 0, st>>>(a);
     if (int rc = launch_status("conv_igemm_f32")) return rc;
     if (tc.splitk > 1) {
         const size_t total = static_cast<size_t>(g.M) * a.ws_ld;
@@ -1933,7 +1782,7 @@ bool tune_tiles(hipStream_t st, const ConvGeom &g, const GatherSpec &gs, int *cf
     size_t wpack_bytes = 0, ws_bytes = 16;
     for (const Cand &cd : keep) {
         const TileCfg &t = kCfgs[cd.cfg];
-        wpack_bytes = std::max(wpack_bytes, static_cast<size_t>(cd.tc.m_tiles) * cd.tc.k_tiles * t.BM * t.BK * 4);
+        wpack_bytes = std::max(wpack_bytes, static_cast<size_t>(cd.tc.m_tiles) * cd.tc.k_tiles * t.BM * t.BK * weight_bytes(cd.cfg));
         ws_bytes = std::max(ws_bytes, partial_bytes_of(cd.tc, g.M, Ntot));
     }
     const size_t y_bytes = static_cast<size_t>(g.y_elems) * 4;
@@ -2098,6 +1947,23 @@ int upload_packed_f32(const float *w, int M, int K, int BM, int BK, int m_tiles,
     return hip_check(hipMemcpy(*out, packed.data(), bytes, hipMemcpyHostToDevice), "hipMemcpy packed weights");
 }
 
+// Packs A[m][k] for conv_split_f32 (pack_split) on the device: the weights
+// travel as floats and are split there (4.7 M of them: 30 ms on the host).
+int upload_packed_split(hipStream_t st, const float *w, int M, int K, int BM, int BK, int m_tiles, int k_tiles,
+                        void **out) {
+    const size_t raw = static_cast<size_t>(M) * K * sizeof(float);
+    if (int rc = hip_check(hipMalloc(out, static_cast<size_t>(m_tiles) * k_tiles * BM * BK * 6),
+                           "hipMalloc packed weights"))
+        return rc;
+    void *tmp = nullptr;
+    if (int rc = hip_check(hipMalloc(&tmp, raw), "hipMalloc weights to pack")) return rc;
+    int rc = hip_check(hipMemcpy(tmp, w, raw, hipMemcpyHostToDevice), "hipMemcpy weights to pack");
+    if (rc == 0) rc = pack_split(st, static_cast<const float *>(tmp), M, K, BM, BK, m_tiles, k_tiles, *out);
+    if (rc == 0) rc = hip_check(hipStreamSynchronize(st), "pack_split");
+    (void)hipFree(tmp);
+    return rc;
+}
+
 // Packs w[m][c][tap] (k = c * taps + tap, the reference's order) for the
 // skinny kernel: k' = tap * C + c in chunks of 64, tile [m_tiles][KC][4 slots
 // g][16 rows][16 t] holding row m, k' = 64 * chunk + 16g + t -- lane (g, row)
@@ -2189,6 +2055,10 @@ static int plan_tiles_and_weights(hipStream_t st, const ConvGeom &g, const Gathe
     } else if (t.thin_mb > 0) {
         if (int rc = upload_packed_thin(w_host, g.M, gs.gather.C, gs.K / gs.gather.C, t.thin_mb, plan->m_tiles,
                                         plan->k_tiles, &plan->wpack))
+            return rc;
+    } else if (t.split_threads > 0) {
+        if (int rc = upload_packed_split(st, w_host, g.M, gs.K, t.BM, t.BK, plan->m_tiles, plan->k_tiles,
+                                         &plan->wpack))
             return rc;
     } else if (int rc = upload_packed_f32(w_host, g.M, gs.K, t.BM, t.BK, plan->m_tiles, plan->k_tiles, &plan->wpack)) {
         return rc;
@@ -2298,7 +2168,7 @@ std::string igemm_name(const ConvPlan *p) {
     if (kCfgs[p->cfg].skinny_waves > 0)
         return std::string("conv_skinny_f32<16x16,w") + std::to_string(kCfgs[p->cfg].skinny_waves) +
                (p->padded ? ",pad" : "") + ">";
-    return std::string("conv_igemm_f32<") + kCfgs[p->cfg].name +
+    return std::string(kCfgs[p->cfg].split_threads > 0 ? "conv_split_f32<" : "conv_igemm_f32<") + kCfgs[p->cfg].name +
            (p->gather.chk ? ",ipad" : p->padded ? ",pad" : "") +
            ",splitk=" + std::to_string(p->splitk) + (p->dp_tiles ? ",dp=" + std::to_string(p->dp_tiles) : "") + ">";
 }
@@ -2386,7 +2256,7 @@ static int use_implicit_padding(ConvPlan *plan) {
     if (!(e && e[0] == '1') && g.C * g.KH * g.KW > 160) return 0;
     const int BK = plan->BK;
     const int K = g.C * g.KH * g.KW;
-    const size_t entries = static_cast<size_t>(plan->Kpad) + 2 * BK;  // as build_koff: two tiles past Kpad
+    const size_t entries = static_cast<size_t>(plan->Kpad) + 3 * BK;  // as build_koff: three tiles past Kpad
     std::vector<int> koff(entries, kOobOffset), ktap(entries, 0x7fff7fff);
     for (int k = 0; k < K; k++) {
         const int c = k / (g.KH * g.KW), r = k % (g.KH * g.KW);

@@ -1,0 +1,377 @@
+// fp32 implicit GEMM on the bf16 matrix cores (conv_split_f32), for the layers
+// large enough to be bound by the fp32 ones.
+//
+// A float is the sum of three bf16 parts (8 + 8 + 8 significant bits), and a
+// product of two floats the sum of nine products of parts, each exact in
+// float32.  The six largest are computed, on v_mfma_f32_32x32x16_bf16, which
+// runs 16 times as many operations a cycle as v_mfma_f32_32x32x2_f32: 2.7
+// times the fp32 rate at the clocks' limit, though at this load the chip
+// holds the matrix cores to about 1.5 PFLOP/s, 1.6 times what the fp32 ones
+// reach.  The three products left out are below 2^-25 of the whole each.
+//
+// Precision: against 64-bit sums of N(0, 1) data the relative error is 5e-8
+// at K = 64, 8.5e-8 at 256 and 2.9e-7 at 2304, where the fp32 MFMA's is
+// 1.4e-7, 2.7e-7 and 8.7e-7: sixteen products are summed before a rounding
+// instead of two, and the five smaller products have an accumulator of their
+// own (in one accumulator all six would round at the sum's size: 7.3e-7 at
+// 2304).  Infinities, NaN, overflows and sums next to the smallest floats are
+// summed again in float32 multiply-adds (below).
+//
+// What bounds it: per 128 x 64 x 32 step a workgroup runs 768 cycles of MFMA
+// a SIMD, loads 24 KB of weights (fragment order, straight to registers) and
+// 8 KB of activations, which it splits (5.5 VALU operations an element) into
+// 12 KB of LDS pieces that every wave reads.  Timed on a 14x14 3x3 layer, 256
+// channels, batch 64 (14.8 GFLOP, 392 tiles on 256 CUs): 101 us; without the
+// activations' loads 90, without splitting them 84, without the weights'
+// loads 75; the fp32 tiles take 117 us.
+#define SPK_SPLIT_DEFINE
+#include "igemm_split.hpp"
+
+namespace spk::kern {
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// x = hi + mid + lo: each the nearest bf16 of what the ones before leave, so
+// the sum is x exactly (three 8-bit significands hold the 24 of a float).
+// Two elements at a time, packed low half first.
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
+    h = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x0, x1}, bf16x2));
+    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+    m = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{r0, r1}, bf16x2));
+    const float s0 = r0 - __uint_as_float(m << 16), s1 = r1 - __uint_as_float(m & 0xffff0000u);
+    l = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{s0, s1}, bf16x2));
+}
+
+// BM x BK tiles [m_tiles][k_tiles], each [BM/32][BK/16][3 parts][64 lanes][8]
+// bf16: lane l of a 32x32x16 step holds row l & 31, k = 8 * (l >> 5) + 0..7 of
+// one part.  One thread per lane and step; ragged edges are zeros.
+__global__ void __launch_bounds__(256) pack_split_kernel(const float *__restrict__ w, int M, int K, int blocks, int steps,
+                                                         int k_tiles, unsigned pieces, uintx4 *__restrict__ out) {
+    const unsigned id = blockIdx.x * 256u + threadIdx.x;
+    if (id >= pieces) return;
+    const unsigned at = id / 64, lane = id & 63;
+    const unsigned step = at % steps, kt = at / (blocks * steps) % k_tiles;
+    const int m = static_cast<int>((at / (k_tiles * blocks * steps) * blocks + at / steps % blocks) * 32 + lane % 32);
+    const int k = static_cast<int>((kt * steps + step) * 16 + lane / 32 * 8);
+    unsigned part[3][8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        float v = m < M && k + j < K ? w[static_cast<size_t>(m) * K + k + j] : 0.0f;
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            // to nearest; the largest floats are cut, so that none becomes
+            // infinite, and infinities and NaN have one part
+            const unsigned u = __float_as_uint(v), mag = u & 0x7fffffffu;
+            const unsigned h = mag > 0x7f800000u    ? u | 0x400000u
+                               : mag >= 0x7f7f8000u ? u
+                                                    : u + 0x7fffu + (u >> 16 & 1);
+            part[p][j] = h >> 16;
+            v = mag >= 0x7f800000u ? 0.0f : v - __uint_as_float(h & 0xffff0000u);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        uintx4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = part[p][2 * e] | part[p][2 * e + 1] << 16;
+        out[(static_cast<size_t>(at) * 3 + p) * 64 + lane] = o;
+    }
+}
+
+// One output's sum over k0 .. k1 - 1 in float32 multiply-adds (the packed
+// parts of a weight add up to it exactly).
+template <int BM, int BK, int MODE>
+__device__ __forceinline__ float plain_sum(const IgemmArgs &a, int m, int n, int k0, int k1) {
+    const int img = n / a.OHW, sp = n - img * a.OHW, oh = sp / a.OW, ow = sp - oh * a.OW;
+    int ihb = oh * a.sh, iwb = ow * a.sw;
+    if (MODE == kModeChk) {
+        ihb -= a.chk_ph;
+        iwb -= a.chk_pw;
+    }
+    const int col = img * a.x_img_stride + ihb * a.Wp + iwb;
+    const unsigned short *w = reinterpret_cast<const unsigned short *>(a.wp);
+    float s = 0.0f;
+    for (int k = k0; k < k1; k++) {
+        if (a.koff[k] == kOobOffset) break;  // past K
+        if (MODE == kModeChk) {
+            const int t = a.ktap[k];
+            if (static_cast<unsigned>(ihb + (t >> 16)) >= static_cast<unsigned>(a.chk_H) ||
+                static_cast<unsigned>(iwb + (t & 0xffff)) >= static_cast<unsigned>(a.chk_W))
+                continue;
+        }
+        const int kt = k / BK, kk = k % BK, ml = m % BM;
+        const size_t at = ((((static_cast<size_t>(m / BM) * a.k_tiles + kt) * (BM / 32) + ml / 32) * (BK / 16) + kk / 16) *
+                               3 * 64 +
+                           (kk % 16 / 8) * 32 + ml % 32) *
+                              8 +
+                          kk % 8;
+        const float wv = __uint_as_float(static_cast<unsigned>(w[at]) << 16) +
+                         (__uint_as_float(static_cast<unsigned>(w[at + 512]) << 16) +
+                          __uint_as_float(static_cast<unsigned>(w[at + 1024]) << 16));
+        s = __builtin_fmaf(wv, a.x[col + a.koff[k] / 4], s);
+    }
+    return s;
+}
+
+}  // namespace
+
+template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WPE, int MODE>
+__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(IgemmArgs a) {
+    constexpr int NT = 64 * WAVES_M * WAVES_N;
+    constexpr int TM = BM / (32 * WAVES_M);
+    constexpr int TN = BN / (32 * WAVES_N);
+    constexpr int Q = BK / 16;           // MFMA k steps per k-tile
+    constexpr int KG = BK / 8;           // 16-byte k groups per plane and column
+    constexpr int KPT = BK * BN / NT;    // B elements per thread per k-tile
+    constexpr int GPT = KPT / 8;         // k groups per thread
+    static_assert(TM >= 1 && TN >= 1 && KPT % 8 == 0 && BN >= 64 && NT % BN == 0, "tile shape");
+
+    // [buffer][plane][k group][column] 16-byte pieces: a thread writes the
+    // pieces of its column, a wave reads 32 columns of two groups, both
+    // contiguous across lanes (no bank conflicts without padding)
+    __shared__ __attribute__((aligned(16))) uintx4 Bs[2][3][KG][BN];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int wm = wave / WAVES_N;
+    const int wn = wave % WAVES_N;
+
+    // tiles, split-K slices and the hybrid schedule as in conv_igemm_f32
+    int bid = blockIdx.x;
+    int slice = blockIdx.y;
+    bool part = a.ws != nullptr;
+    if (a.dp_tiles > 0) {
+        if (bid < a.dp_tiles) {
+            if ((a.dp_tiles & 7) == 0) bid = (bid & 7) * (a.dp_tiles >> 3) + (bid >> 3);
+            part = false;
+        } else {
+            const int r = bid - a.dp_tiles;
+            bid = a.dp_tiles + r / a.rem_split;
+            slice = r - (r / a.rem_split) * a.rem_split;
+        }
+    } else {
+        const int nb = gridDim.x;
+        if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
+    }
+    const int mt = bid % a.m_tiles;
+    const int nt = bid / a.m_tiles;
+    const int kt0 = part ? slice * a.kt_per_split : 0;
+    const int kt1 = part ? min(kt0 + a.kt_per_split, a.k_tiles) : a.k_tiles;
+    if (kt0 >= kt1) return;  // empty split-K slice
+
+    const int bcol = tid % BN;
+    const int bgrp = __builtin_amdgcn_readfirstlane(tid / BN);  // wave-uniform: BN >= 64
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.x), static_cast<short>(0), a.x_bytes, kBufferWord3);
+    const int row = lane & 31;
+    const int half = lane >> 5;
+
+    int col = kOobOffset;
+    int ihb = 0x40000000, iwb = 0;  // kModeChk: the column's input row / column at tap (0, 0)
+    {
+        const int n = nt * BN + bcol;
+        if (n < a.Ntot) {
+            const int img = n / a.OHW;
+            const int sp = n - img * a.OHW;
+            const int oh = sp / a.OW;
+            const int ow = sp - oh * a.OW;
+            if constexpr (MODE == kModeChk) {
+                ihb = oh * a.sh - a.chk_ph;
+                iwb = ow * a.sw - a.chk_pw;
+                col = (img * a.x_img_stride + ihb * a.Wp + iwb) * 4;  // may be negative: used only in bounds
+            } else {
+                col = (img * a.x_img_stride + oh * a.sh * a.Wp + ow * a.sw) * 4;
+            }
+        }
+    }
+
+    // A: [m_tile][k_tile][32-row block][k step][part][lane] 16-byte pieces
+    const bf16x8 *const wbase = reinterpret_cast<const bf16x8 *>(a.wp) +
+                                (static_cast<size_t>(mt) * a.k_tiles * (BM / 32) + wm * TM) * (Q * 3 * 64) + lane;
+    bf16x8 a0[TM][Q][3], a1[TM][Q][3];
+    float br0[KPT], br1[KPT];
+
+    auto load_a = [&](int kt, bf16x8 (&ax)[TM][Q][3]) __attribute__((always_inline)) {
+        const bf16x8 *src = wbase + static_cast<size_t>(min(kt, a.k_tiles - 1)) * ((BM / 32) * Q * 3 * 64);
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) ax[i][q][p] = src[((i * Q + q) * 3 + p) * 64];
+    };
+    // The k offsets are read one tile ahead of the loads that use them (the
+    // table has three tiles of out-of-range entries past K).
+    int ko[KPT];
+    auto load_ko = [&](int kt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < KPT; j++) ko[j] = a.koff[kt * BK + bgrp * KPT + j];
+    };
+    auto load_b = [&](int kt, float (&br)[KPT]) __attribute__((always_inline)) {
+        if constexpr (MODE == kModeKvec) {
+#pragma unroll
+            for (int j = 0; j < KPT; j += 4) {
+                const floatx4 v =
+                    __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xrs, col, ko[j], 0));
+                br[j] = v[0];
+                br[j + 1] = v[1];
+                br[j + 2] = v[2];
+                br[j + 3] = v[3];
+            }
+        } else if constexpr (MODE == kModeChk) {
+            const int *tp = a.ktap + kt * BK + bgrp * KPT;
+#pragma unroll
+            for (int j = 0; j < KPT; j++) {
+                const int t = tp[j];
+                const bool in = static_cast<unsigned>(ihb + (t >> 16)) < static_cast<unsigned>(a.chk_H) &&
+                                static_cast<unsigned>(iwb + (t & 0xffff)) < static_cast<unsigned>(a.chk_W);
+                br[j] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(xrs, in ? col + ko[j] : kOobOffset, 0, 0));
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < KPT; j++)
+                br[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, col, ko[j], 0));
+        }
+        load_ko(kt + 1);
+    };
+    auto store_b = [&](int buf, const float (&br)[KPT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < GPT; g++) {
+            uintx4 h, m, l;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                unsigned hv, mv, lv;
+                split_pair(br[g * 8 + 2 * e], br[g * 8 + 2 * e + 1], hv, mv, lv);
+                h[e] = hv;
+                m[e] = mv;
+                l[e] = lv;
+            }
+            Bs[buf][0][bgrp * GPT + g][bcol] = h;
+            Bs[buf][1][bgrp * GPT + g][bcol] = m;
+            Bs[buf][2][bgrp * GPT + g][bcol] = l;
+        }
+    };
+
+    floatx16 acc[TM][TN], sml[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = sml[i][j][r] = 0.0f;
+
+    auto frag_b = [&](int buf, int q, int p, bf16x8 (&bf)[TN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            bf[j] = __builtin_bit_cast(bf16x8, Bs[buf][p][2 * q + half][(wn * TN + j) * 32 + row]);
+    };
+    // one product of parts over the wave's blocks
+    auto mma = [&](const bf16x8 (&ax)[TM][Q][3], int q, int pa, const bf16x8 (&bf)[TN],
+                   floatx16 (&c)[TM][TN]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                c[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax[i][q][pa], bf[j], c[i][j], 0, 0, 0);
+    };
+    // The five products of 2^-8 and below keep a sum of their own: added one
+    // by one to the large one each would round at its size.
+    auto compute = [&](int buf, const bf16x8 (&ac)[TM][Q][3], auto &&between) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            bf16x8 bh[TN], bm[TN], bl[TN];
+            frag_b(buf, q, 0, bh);
+            frag_b(buf, q, 1, bm);
+            frag_b(buf, q, 2, bl);
+            mma(ac, q, 0, bh, acc);
+            mma(ac, q, 2, bh, sml);
+            if (q == 0) between();
+            mma(ac, q, 1, bh, sml);
+            mma(ac, q, 1, bm, sml);
+            mma(ac, q, 0, bm, sml);
+            mma(ac, q, 0, bl, sml);
+        }
+    };
+    auto step = [&](int kt, int buf, const bf16x8 (&ac)[TM][Q][3], bf16x8 (&an)[TM][Q][3], const float (&bnx)[KPT],
+                    float (&bfree)[KPT]) __attribute__((always_inline)) {
+        load_b(kt + 2, bfree);
+        load_a(kt + 1, an);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(buf, ac, [&]() __attribute__((always_inline)) { store_b(buf ^ 1, bnx); });
+        __syncthreads();
+    };
+
+    load_ko(kt0);
+    load_b(kt0, br0);
+    load_b(kt0 + 1, br1);
+    load_a(kt0, a0);
+    store_b(0, br0);
+    __syncthreads();
+    int kt = kt0;
+    // tiles past kt1 are loaded and ignored, which keeps the loop free of
+    // data-dependent branches
+    for (; kt + 1 < kt1; kt += 2) {
+        step(kt, 0, a0, a1, br1, br0);
+        step(kt + 1, 1, a1, a0, br0, br1);
+    }
+    if (kt < kt1) compute(0, a0, []() {});
+
+    // An infinite input or product has parts of both signs, whose sum is not
+    // what a float32 sum gives, and the parts of values near the smallest
+    // float round to zero: such outputs are summed again without parts.
+    constexpr int OUTS = TM * TN * 16;
+    static_assert(OUTS <= 128, "two masks");
+    unsigned long long odd0 = 0, odd1 = 0;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            acc[i][j] += sml[i][j];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float v = __builtin_fabsf(acc[i][j][r]);
+                const int e = (i * TN + j) * 16 + r;
+                const bool odd = !(v < __builtin_inff()) || (v < 0x1p-90f && v != 0.0f);
+                (e < 64 ? odd0 : odd1) |= static_cast<unsigned long long>(odd) << (e & 63);
+            }
+        }
+    if (odd0 | odd1) {
+        for (int e = 0; e < OUTS; e++) {
+            if (!((e < 64 ? odd0 : odd1) >> (e & 63) & 1)) continue;
+            const int m = mt * BM + (wm * TM + e / (TN * 16)) * 32 + 4 * half + e % 16 / 4 * 8 + e % 4;
+            const int n = nt * BN + (wn * TN + e / 16 % TN) * 32 + row;
+            if (m >= a.M || n >= a.Ntot) continue;
+            const float v = plain_sum<BM, BK, MODE>(a, m, n, kt0 * BK, kt1 * BK);
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++)
+                        if (e == (i * TN + j) * 16 + r) acc[i][j][r] = v;
+        }
+    }
+    igemm_epilogue<BM, BN, 32, TM, TN>(a, acc, mt, nt, wm, wn, lane, part, slice);
+}
+
+int pack_split(hipStream_t st, const float *w, int M, int K, int BM, int BK, int m_tiles, int k_tiles, void *out) {
+    const size_t pieces = static_cast<size_t>(m_tiles) * k_tiles * (BM / 32) * (BK / 16) * 64;
+    if (pieces >= (size_t(1) << 31)) return SPKV2_E_UNSUPPORTED;
+    hipLaunchKernelGGL(pack_split_kernel, dim3(blocks_for(pieces, 256)), dim3(256), 0, st, w, M, K, BM / 32, BK / 16,
+                       k_tiles, static_cast<unsigned>(pieces), static_cast<uintx4 *>(out));
+    return launch_status("pack_split");
+}
+
+#define SPLIT(BM, BN, BK, WM, WN, WPE, EFF)                                                  \
+    template __global__ void conv_split_f32<BM, BN, BK, WM, WN, WPE, kModePlain>(IgemmArgs); \
+    template __global__ void conv_split_f32<BM, BN, BK, WM, WN, WPE, kModeKvec>(IgemmArgs);  \
+    template __global__ void conv_split_f32<BM, BN, BK, WM, WN, WPE, kModeChk>(IgemmArgs);
+SPK_SPLIT_TILES(SPLIT)
+#undef SPLIT
+
+}  // namespace spk::kern
