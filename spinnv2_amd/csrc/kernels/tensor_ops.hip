@@ -254,24 +254,32 @@ __device__ __forceinline__ void topk_sift(HeapPair *h, int n, int i, int largest
     h[i] = e;
 }
 
-// The reference's insertion (tensor/topk.c:87-92 and 97-101): e replaces
-// the root and is sifted down (topk_sift's rule), two levels per round trip
-// to LDS (a node's children and grandchildren are read together; only the
-// path's nodes are written).  Returns the value left at the root.
-__device__ __forceinline__ float topk_sift_root(HeapPair *h, int n, HeapPair e, int largest) {
-    auto above = [&](float a, float b) { return largest ? (a < b) : (a > b); };  // a belongs above b
-    int i = 0;
-    float rootv = e.v;
-    for (;;) {
-        const int l = 2 * i + 1;
-        if (l >= n) break;
-        const int g = 2 * l + 1;  // children of l: g, g + 1; of l + 1: g + 2, g + 3
-        const HeapPair c0 = h[l], c1 = h[min(l + 1, n - 1)];
-        const HeapPair g0 = h[min(g, n - 1)], g1 = h[min(g + 1, n - 1)];
-        const HeapPair g2 = h[min(g + 2, n - 1)], g3 = h[min(g + 3, n - 1)];
-        int m = i;
+// The reference's insertions (tensor/topk.c:87-92 and 97-101), where e
+// replaces the root of a heap of n and is sifted down (topk_sift's rule), as
+// a pipeline of one wave: lane L carries the insertion that has reached level
+// L, and a step moves every insertion one level down.  A step at level L reads
+// level L + 1 and writes level L, so an insertion may enter every second step
+// and finds the heap as the ones before it leave it.  A step is one LDS round
+// trip and some 20 operations; sifting one insertion after the other in one
+// lane took about 1.5 us each, the depth of the heap in round trips.
+struct HeapPipe {
+    HeapPair *h;
+    int n, largest;
+    HeapPair e{0.0f, 0u};
+    int node = 0, active = 0;
+
+    // lane 0's value moves to lane 1, ...; lane 0 becomes `first`
+    static __device__ __forceinline__ int down(int v, int first) {
+        return __builtin_amdgcn_update_dpp(first, v, 0x111 /* row_shr:1 */, 0xf, 0xf, false);
+    }
+    // returns the value at the root (of an insertion that enters this step)
+    __device__ __forceinline__ float step() {
+        auto above = [&](float a, float b) { return largest ? (a < b) : (a > b); };  // a belongs above b
+        const int l = 2 * node + 1;
+        const HeapPair c0 = h[min(l, n - 1)], c1 = h[min(l + 1, n - 1)];
+        int m = node;
         HeapPair mv = e;
-        if (above(c0.v, mv.v)) {
+        if (l < n && above(c0.v, mv.v)) {
             m = l;
             mv = c0;
         }
@@ -279,31 +287,34 @@ __device__ __forceinline__ float topk_sift_root(HeapPair *h, int n, HeapPair e, 
             m = l + 1;
             mv = c1;
         }
-        if (m == i) break;
-        h[i] = mv;
-        if (i == 0) rootv = mv.v;
-        const bool left = m == l;
-        i = m;
-        const int l2 = 2 * i + 1;
-        if (l2 >= n) break;
-        const HeapPair d0 = left ? g0 : g2, d1 = left ? g1 : g3;
-        m = i;
-        mv = e;
-        if (above(d0.v, mv.v)) {
-            m = l2;
-            mv = d0;
-        }
-        if (l2 + 1 < n && above(d1.v, mv.v)) {
-            m = l2 + 1;
-            mv = d1;
-        }
-        if (m == i) break;
-        h[i] = mv;
-        i = m;
+        if (active) h[node] = mv;
+        active = down(active && m != node, 0);
+        e.v = __int_as_float(down(__float_as_int(e.v), 0));
+        e.idx = static_cast<uint32_t>(down(static_cast<int>(e.idx), 0));
+        node = down(m, 0);
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mv.v), 0));
     }
-    h[i] = e;
-    return rootv;
-}
+    // the wave's 64 elements from index d0 on, in order: those that are
+    // candidates and better than the root when their turn comes enter
+    __device__ __forceinline__ void feed(float v, bool cand, int d0, int lane, float &root) {
+        unsigned long long m = __ballot(cand && (largest ? (v > root) : (v < root)));
+        while (m) {
+            const int j = __ffsll(static_cast<long long>(m)) - 1;
+            const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+            if (lane == 0) {
+                e = HeapPair{vj, static_cast<uint32_t>(d0 + j)};
+                node = 0;
+                active = 1;
+            }
+            root = step();
+            step();
+            m = __ballot(cand && lane > j && (largest ? (v > root) : (v < root)));
+        }
+    }
+    __device__ __forceinline__ void drain() {
+        while (__ballot(active)) step();
+    }
+};
 
 constexpr int kTopkThreads = 1024;
 constexpr int kTopkWaves = kTopkThreads / 64;
@@ -344,9 +355,9 @@ __device__ __forceinline__ uint32_t topk_scan(uint32_t v, uint32_t *wsum, int ti
 //   * the heap's root only gets better as elements enter, so an element no
 //     better than the root after heapify never enters: all threads mark the
 //     others first (a bit per element), and one wave walks only the marked
-//     ones in element order, testing 64 at a time against the current root;
-//     lane 0 inserts the first that enters and the rest are re-tested
-//     against the new root.
+//     ones in element order, testing 64 at a time against the current root:
+//     the first that enters goes into the pipeline of insertions (HeapPipe)
+//     and the rest are re-tested against the new root.
 template <bool STAGED>
 __global__ void __launch_bounds__(kTopkThreads) topk_kernel(const float *__restrict__ x, float *__restrict__ values,
                                                             float *__restrict__ indices, size_t inner, int dim, int k,
@@ -473,6 +484,7 @@ __global__ void __launch_bounds__(kTopkThreads) topk_kernel(const float *__restr
             __syncthreads();
             if (wave == 0) {
                 float root = root0;
+                HeapPipe pipe{heap, k, largest};
                 for (int b0 = 0; b0 < nblk; b0 += 64) {
                     const unsigned long long mine = b0 + lane < nblk ? cmask[b0 + lane] : 0ull;
                     unsigned long long nz = __ballot(mine != 0ull);
@@ -482,35 +494,20 @@ __global__ void __launch_bounds__(kTopkThreads) topk_kernel(const float *__restr
                         const unsigned long long cm = __shfl(mine, jb);
                         const int d0 = k + 64 * (b0 + jb);
                         const bool cand = (cm >> lane) & 1ull;
-                        const float v = cand ? rowbuf[d0 + lane] : 0.0f;
-                        unsigned long long m = __ballot(cand && (largest ? (v > root) : (v < root)));
-                        while (m) {
-                            const int j = __ffsll(static_cast<long long>(m)) - 1;
-                            const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-                            float r = 0.0f;
-                            if (lane == 0) r = topk_sift_root(heap, k, HeapPair{vj, static_cast<uint32_t>(d0 + j)}, largest);
-                            root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 0));
-                            m = __ballot(cand && lane > j && (largest ? (v > root) : (v < root)));
-                        }
+                        pipe.feed(cand ? rowbuf[d0 + lane] : 0.0f, cand, d0, lane, root);
                     }
                 }
+                pipe.drain();
             }
         } else if (wave == 0) {  // rows beyond the LDS: the same walk over every element, from memory
             float root = root0;
+            HeapPipe pipe{heap, k, largest};
             for (int d0 = k; d0 < dim; d0 += 64) {
                 const int d = d0 + lane;
                 const bool live = d < dim;
-                const float v = live ? x[base + static_cast<size_t>(d) * inner] : 0.0f;
-                unsigned long long m = __ballot(live && (largest ? (v > root) : (v < root)));
-                while (m) {
-                    const int j = __ffsll(static_cast<long long>(m)) - 1;
-                    const float vj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-                    float r = 0.0f;
-                    if (lane == 0) r = topk_sift_root(heap, k, HeapPair{vj, static_cast<uint32_t>(d0 + j)}, largest);
-                    root = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 0));
-                    m = __ballot(live && lane > j && (largest ? (v > root) : (v < root)));
-                }
+                pipe.feed(live ? x[base + static_cast<size_t>(d) * inner] : 0.0f, live, d0, lane, root);
             }
+            pipe.drain();
         }
         __syncthreads();
         for (int i = tid; i < k; i += kTopkThreads)
