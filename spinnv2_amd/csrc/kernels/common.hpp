@@ -32,6 +32,22 @@ __device__ __forceinline__ float apply_act(float v, int act) {
     return v;
 }
 
+// n / d for 0 <= n < 2^31 with (m, s) from div_magic(d): m = ceil(2^s / d),
+// s = 31 + ceil(log2 d), so n m / 2^s is within 2^-ceil(log2 d) <= 1/d of
+// n / d and its floor is exact.  One 32 x 32 -> 64 multiply and a shift
+// instead of a division sequence.
+__device__ __forceinline__ int div_fast(int n, unsigned m, int s) {
+    return static_cast<int>((static_cast<uint64_t>(static_cast<unsigned>(n)) * m) >> s);
+}
+
+// (m, s) of div_fast for divisor d >= 1 (dividends below 2^31)
+inline void div_magic(unsigned d, unsigned *m, int *s) {
+    int l = 0;
+    while ((uint64_t(1) << l) < d) l++;
+    *s = 31 + l;
+    *m = static_cast<unsigned>(((uint64_t(1) << *s) + d - 1) / d);
+}
+
 inline size_t elem_count(const Spkv2TensorRecord *r) {
     size_t n = 1;
     for (uint16_t i = 0; i < r->rank; i++) n *= r->shape[i];

@@ -902,35 +902,57 @@ __global__ void __launch_bounds__(256) splitk_epilogue(const float *__restrict__
 }
 
 // Zero-padded copy of an NCHW tensor: planes of H x W placed at (pt, pl) in
-// planes of Hp x Wp, halo written as zeros.  grid.y strides over planes,
-// grid.x over the elements of a plane (32-bit index math), so small
-// batches still spread over the GPU.
-__global__ void __launch_bounds__(256) pad_nchw(const float *__restrict__ x, float *__restrict__ xp, unsigned planes,
-                                                unsigned C, size_t x_img, int H, int W, int Hp, int Wp, int pt,
-                                                int pl) {
-    const unsigned plane_sz = static_cast<unsigned>(Hp * Wp);
-    for (unsigned plane = blockIdx.y; plane < planes; plane += gridDim.y) {
-        // images x_img elements apart (more than C planes: a channel slice)
-        const float *src = x + (plane / C) * x_img + static_cast<size_t>(plane % C) * H * W;
-        float *dst = xp + static_cast<size_t>(plane) * plane_sz;
-        for (unsigned r = blockIdx.x * 256 + threadIdx.x; r < plane_sz; r += gridDim.x * 256) {
-            const int hq = static_cast<int>(r / static_cast<unsigned>(Wp));
-            const int h = hq - pt, w = static_cast<int>(r) - hq * Wp - pl;
-            dst[r] = (static_cast<unsigned>(h) < static_cast<unsigned>(H) && static_cast<unsigned>(w) < static_cast<unsigned>(W))
-                         ? src[h * W + w]
-                         : 0.0f;
+// planes of Hp x Wp, halo written as zeros.  Memory-bound: each thread writes
+// four consecutive elements of the padded tensor (16 bytes), with its four
+// loads in flight together; the first one's plane, row and column come from
+// multiply-and-shift divisions and the others' by carrying (one element per
+// thread with divisions of its own: 12.4 us for 64 x 256 planes of 14 x 14,
+// 8.0 us so).
+struct PadArgs {
+    const float *__restrict__ x;
+    float *__restrict__ xp;
+    unsigned total;  // padded elements
+    int C, H, W, Hp, Wp, pt, pl;
+    size_t x_img;  // elements between images: more than C planes for a channel slice
+    unsigned plane_m, wp_m, c_m;
+    int plane_s, wp_s, c_s;
+};
+__global__ void __launch_bounds__(256) pad_nchw(PadArgs a) {
+    const unsigned i0 = (blockIdx.x * 256u + threadIdx.x) * 4u;
+    if (i0 >= a.total) return;
+    const int plane_sz = a.Hp * a.Wp;
+    int plane = div_fast(static_cast<int>(i0), a.plane_m, a.plane_s);
+    const int r = static_cast<int>(i0) - plane * plane_sz;
+    int hq = div_fast(r, a.wp_m, a.wp_s);
+    int wq = r - hq * a.Wp;
+    int img = div_fast(plane, a.c_m, a.c_s);
+    int c = plane - img * a.C;
+    floatx4 v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int h = hq - a.pt, w = wq - a.pl;
+        const bool in = static_cast<unsigned>(h) < static_cast<unsigned>(a.H) &&
+                        static_cast<unsigned>(w) < static_cast<unsigned>(a.W) && i0 + e < a.total;
+        v[e] = in ? a.x[static_cast<size_t>(img) * a.x_img + (static_cast<size_t>(c) * a.H + h) * a.W + w] : 0.0f;
+        if (++wq == a.Wp) {
+            wq = 0;
+            if (++hq == a.Hp) {
+                hq = 0;
+                if (++c == a.C) {
+                    c = 0;
+                    img++;
+                }
+            }
         }
     }
+    if (i0 + 4 <= a.total) {
+        // a caller's scratch arena need not be aligned to more than a float
+        typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+        *reinterpret_cast<floatx4_any *>(a.xp + i0) = v;
+    } else {
+        for (unsigned e = 0; i0 + e < a.total; e++) a.xp[i0 + e] = v[e];
+    }
 }
-
-// grid of a per-plane kernel: x covers `per_plane` elements with 256-thread
-// blocks, y the planes (capped; the kernels stride over the rest)
-inline dim3 plane_grid(size_t per_plane, size_t planes) {
-    const size_t gx = std::min<size_t>((per_plane + 255) / 256, 1024);
-    const size_t gy = std::min<size_t>(planes, 65535);
-    return dim3(static_cast<unsigned>(gx == 0 ? 1 : gx), static_cast<unsigned>(gy == 0 ? 1 : gy));
-}
-
 
 // ------------------------------------------------------------ direct kernel
 
@@ -2219,9 +2241,22 @@ static int run_igemm_impl(Spkv2Context *ctx, const ConvPlan *p, const float *x, 
     } else if (p->padded) {
         float *xp = reinterpret_cast<float *>(wsb);
         const unsigned planes = static_cast<unsigned>(g.N * g.C);
-        hipLaunchKernelGGL(pad_nchw, plane_grid(static_cast<size_t>(p->Hp) * p->Wp, planes), dim3(256), 0,
-                           ctx->stream, x, xp, planes, static_cast<unsigned>(g.C), static_cast<size_t>(x_img_stride),
-                           g.H, g.W, p->Hp, p->Wp, p->pt, p->pl);
+        PadArgs pa{};
+        pa.x = x;
+        pa.xp = xp;
+        pa.total = planes * static_cast<unsigned>(p->Hp * p->Wp);  // below 2^29 (plan_igemm_f32)
+        pa.C = g.C;
+        pa.H = g.H;
+        pa.W = g.W;
+        pa.Hp = p->Hp;
+        pa.Wp = p->Wp;
+        pa.pt = p->pt;
+        pa.pl = p->pl;
+        pa.x_img = static_cast<size_t>(x_img_stride);
+        div_magic(static_cast<unsigned>(p->Hp * p->Wp), &pa.plane_m, &pa.plane_s);
+        div_magic(static_cast<unsigned>(p->Wp), &pa.wp_m, &pa.wp_s);
+        div_magic(static_cast<unsigned>(g.C), &pa.c_m, &pa.c_s);
+        hipLaunchKernelGGL(pad_nchw, dim3((pa.total / 4 + 256) / 256), dim3(256), 0, ctx->stream, pa);
         if (int rc = launch_status("pad_nchw")) return rc;
         xs = xp;
         x_bytes = static_cast<int>(static_cast<size_t>(planes) * p->Hp * p->Wp * 4);
