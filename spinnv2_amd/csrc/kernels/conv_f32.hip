@@ -1617,6 +1617,10 @@ static int launch_igemm(hipStream_t st, int cfg, const TileCounts &tc, const Con
     a.chk_W = gg.chk_W;
     a.chk_ph = gg.chk_ph;
     a.chk_pw = gg.chk_pw;
+    a.chk_KH = g.KH;
+    a.chk_KW = g.KW;
+    a.chk_dh = g.dh;
+    a.chk_dw = g.dw;
     // 16-byte B loads need a 16-byte aligned source (a caller-bound input may not be)
     const bool kvec = gg.kvec && (reinterpret_cast<uintptr_t>(xs) & 15) == 0;
     (kvec ? t.kernel_kvec : gg.chk ? t.kernel_chk : t.kernel)<<<grid, dim3(cfg_threads(cfg)), 0, st>>>(a);
@@ -2279,7 +2283,13 @@ static int run_igemm_impl(Spkv2Context *ctx, const ConvPlan *p, const float *x, 
 // element cost more than the copy saves (a 64-channel 3x3 conv at 80x80,
 // batch 16: 170 against 124 us with its copy), so they keep the copy; so
 // do the skinny kernel (it reads a padded input) and inputs 16384 or more
-// rows or columns tall (the tap table packs a tap into 16 bits).
+// rows or columns tall (the tap table packs a tap into 16 bits).  The tiles
+// on bf16 parts check a tap with one and and one compare (tap_mask), and take
+// the checks with 128 rows, which share an element's check, always (the 14x14
+// 3x3 layer, 256 channels: batch 64 110 us with the copy, 109 without, batch 8
+// 33.4 and 31.1, 72 to 100 channels at 75x57 stride 2 29.9 and 24.4), with
+// fewer rows while the copy costs more than about 3% of the layer: below 6
+// GFLOP (64 rows, batch 64: 137 and 141 us; batch 8: 36.9 and 33.9).
 // SPKV2_IMPLICIT_PAD=0 keeps the copy everywhere, =1 takes the checks
 // wherever they apply.
 static int use_implicit_padding(ConvPlan *plan) {
@@ -2288,16 +2298,19 @@ static int use_implicit_padding(ConvPlan *plan) {
     if (g.H >= 16384 || g.W >= 16384 || (g.KH - 1) * g.dh >= 32768 || (g.KW - 1) * g.dw >= 32768) return 0;
     const char *e = getenv("SPKV2_IMPLICIT_PAD");
     if (e && e[0] == '0') return 0;
-    if (!(e && e[0] == '1') && g.C * g.KH * g.KW > 160) return 0;
+    const bool parts = kCfgs[plan->cfg].split_threads > 0;
+    if (parts && (g.KH > 15 || g.KW > 15)) return 0;  // its tap table has 15 bits a side
+    const double gflop = 2e-9 * static_cast<double>(g.y_elems) * g.C * g.KH * g.KW;
+    if (!(e && e[0] == '1') && g.C * g.KH * g.KW > 160 && !(parts && (plan->BM >= 128 || gflop < 6.0))) return 0;
     const int BK = plan->BK;
     const int K = g.C * g.KH * g.KW;
     const size_t entries = static_cast<size_t>(plan->Kpad) + 3 * BK;  // as build_koff: three tiles past Kpad
-    std::vector<int> koff(entries, kOobOffset), ktap(entries, 0x7fff7fff);
+    std::vector<int> koff(entries, kOobOffset), ktap(entries, parts ? -1 : 0x7fff7fff);
     for (int k = 0; k < K; k++) {
         const int c = k / (g.KH * g.KW), r = k % (g.KH * g.KW);
         const int th = (r / g.KW) * g.dh, tw = (r % g.KW) * g.dw;
         koff[k] = ((c * g.H + th) * g.W + tw) * 4;
-        ktap[k] = (th << 16) | tw;
+        ktap[k] = parts ? (1 << (r / g.KW)) | (1 << (16 + r % g.KW)) : (th << 16) | tw;
     }
     void *kt = nullptr, *tt = nullptr;
     if (int rc = upload_koff(koff, &kt)) return rc;

@@ -81,6 +81,20 @@ __global__ void __launch_bounds__(256) pack_split_kernel(const float *__restrict
     }
 }
 
+// Implicit padding: bit kh of the result is set when tap row kh of the column
+// whose tap (0, 0) is at (ih, iw) lies inside the input, bit 16 + kw when tap
+// column kw does.  The table holds bits kh and 16 + kw for each k, so an
+// element's check is one and, one compare.
+__device__ __forceinline__ unsigned tap_mask(const IgemmArgs &a, int ih, int iw) {
+    unsigned v = 0;
+    for (int t = 0; t < a.chk_KH; t++)
+        v |= static_cast<unsigned>(static_cast<unsigned>(ih + t * a.chk_dh) < static_cast<unsigned>(a.chk_H)) << t;
+    for (int t = 0; t < a.chk_KW; t++)
+        v |= static_cast<unsigned>(static_cast<unsigned>(iw + t * a.chk_dw) < static_cast<unsigned>(a.chk_W))
+             << (16 + t);
+    return v;
+}
+
 // One output's sum over k0 .. k1 - 1 in float32 multiply-adds (the packed
 // parts of a weight add up to it exactly).
 template <int BM, int BK, int MODE>
@@ -92,15 +106,15 @@ __device__ __forceinline__ float plain_sum(const IgemmArgs &a, int m, int n, int
         iwb -= a.chk_pw;
     }
     const int col = img * a.x_img_stride + ihb * a.Wp + iwb;
+    const unsigned valid = MODE == kModeChk ? tap_mask(a, ihb, iwb) : 0u;
     const unsigned short *w = reinterpret_cast<const unsigned short *>(a.wp);
     float s = 0.0f;
     for (int k = k0; k < k1; k++) {
         if (a.koff[k] == kOobOffset) break;  // past K
+        bool in = true;  // taps outside the input are zeros
         if (MODE == kModeChk) {
-            const int t = a.ktap[k];
-            if (static_cast<unsigned>(ihb + (t >> 16)) >= static_cast<unsigned>(a.chk_H) ||
-                static_cast<unsigned>(iwb + (t & 0xffff)) >= static_cast<unsigned>(a.chk_W))
-                continue;
+            const unsigned t = static_cast<unsigned>(a.ktap[k]);
+            in = (valid & t) == t;
         }
         const int kt = k / BK, kk = k % BK, ml = m % BM;
         const size_t at = ((((static_cast<size_t>(m / BM) * a.k_tiles + kt) * (BM / 32) + ml / 32) * (BK / 16) + kk / 16) *
@@ -111,7 +125,7 @@ __device__ __forceinline__ float plain_sum(const IgemmArgs &a, int m, int n, int
         const float wv = __uint_as_float(static_cast<unsigned>(w[at]) << 16) +
                          (__uint_as_float(static_cast<unsigned>(w[at + 512]) << 16) +
                           __uint_as_float(static_cast<unsigned>(w[at + 1024]) << 16));
-        s = __builtin_fmaf(wv, a.x[col + a.koff[k] / 4], s);
+        s = __builtin_fmaf(wv, in ? a.x[col + a.koff[k] / 4] : 0.0f, s);
     }
     return s;
 }
@@ -165,13 +179,18 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
 
     const int bcol = tid % BN;
     const int bgrp = __builtin_amdgcn_readfirstlane(tid / BN);  // wave-uniform: BN >= 64
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(a.x), static_cast<short>(0), a.x_bytes, kBufferWord3);
     const int row = lane & 31;
     const int half = lane >> 5;
 
+    // kModeChk: tap (0, 0) of a column may lie up to `before` bytes ahead of
+    // the input; offsets count from there, so that none is negative (no load
+    // goes there: its taps are not valid)
+    const int before = MODE == kModeChk ? (a.chk_ph * a.Wp + a.chk_pw) * 4 : 0;
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char *>(reinterpret_cast<const char *>(a.x) - before), static_cast<short>(0), a.x_bytes + before,
+        kBufferWord3);
     int col = kOobOffset;
-    int ihb = 0x40000000, iwb = 0;  // kModeChk: the column's input row / column at tap (0, 0)
+    unsigned valid = 0;  // kModeChk: the column's taps inside the input
     {
         const int n = nt * BN + bcol;
         if (n < a.Ntot) {
@@ -179,13 +198,9 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
             const int sp = n - img * a.OHW;
             const int oh = sp / a.OW;
             const int ow = sp - oh * a.OW;
-            if constexpr (MODE == kModeChk) {
-                ihb = oh * a.sh - a.chk_ph;
-                iwb = ow * a.sw - a.chk_pw;
-                col = (img * a.x_img_stride + ihb * a.Wp + iwb) * 4;  // may be negative: used only in bounds
-            } else {
-                col = (img * a.x_img_stride + oh * a.sh * a.Wp + ow * a.sw) * 4;
-            }
+            // from `before` ahead of the input, tap (0, 0) is at row oh * sh
+            col = (img * a.x_img_stride + oh * a.sh * a.Wp + ow * a.sw) * 4;
+            if constexpr (MODE == kModeChk) valid = tap_mask(a, oh * a.sh - a.chk_ph, ow * a.sw - a.chk_pw);
         }
     }
 
@@ -207,9 +222,13 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
     // The k offsets are read one tile ahead of the loads that use them (the
     // table has three tiles of out-of-range entries past K).
     int ko[KPT];
+    unsigned tap[MODE == kModeChk ? KPT : 1];
     auto load_ko = [&](int kt) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < KPT; j++) ko[j] = a.koff[kt * BK + bgrp * KPT + j];
+        for (int j = 0; j < KPT; j++) {
+            ko[j] = a.koff[kt * BK + bgrp * KPT + j];
+            if constexpr (MODE == kModeChk) tap[j] = static_cast<unsigned>(a.ktap[kt * BK + bgrp * KPT + j]);
+        }
     };
     auto load_b = [&](int kt, float (&br)[KPT]) __attribute__((always_inline)) {
         if constexpr (MODE == kModeKvec) {
@@ -223,15 +242,10 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
                 br[j + 3] = v[3];
             }
         } else if constexpr (MODE == kModeChk) {
-            const int *tp = a.ktap + kt * BK + bgrp * KPT;
 #pragma unroll
-            for (int j = 0; j < KPT; j++) {
-                const int t = tp[j];
-                const bool in = static_cast<unsigned>(ihb + (t >> 16)) < static_cast<unsigned>(a.chk_H) &&
-                                static_cast<unsigned>(iwb + (t & 0xffff)) < static_cast<unsigned>(a.chk_W);
-                br[j] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_raw_buffer_load_b32(xrs, in ? col + ko[j] : kOobOffset, 0, 0));
-            }
+            for (int j = 0; j < KPT; j++)
+                br[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                      xrs, (valid & tap[j]) == tap[j] ? col : kOobOffset, ko[j], 0));
         } else {
 #pragma unroll
             for (int j = 0; j < KPT; j++)

@@ -49,6 +49,7 @@ struct IgemmArgs {
     // 0x7fff7fff past K), the unpadded input's extent and the padding
     const int *__restrict__ ktap;
     int chk_H, chk_W, chk_ph, chk_pw;
+    int chk_KH, chk_KW, chk_dh, chk_dw;  // conv_split_f32: its ktap entry is bits kh and 16 + kw, all ones past K
     int th_steps;  // thin kernel: K / 4 MFMA steps (k' = tap * sk_C + c)
     // row-window kernel: the input window's geometry (GatherGeom's win_*)
     int win_KH, win_len, win_shift, win_owb, win_OH, win_dw;

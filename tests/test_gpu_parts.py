@@ -120,10 +120,12 @@ def test_parts_error_is_below_the_fp32_tiles(gpu, monkeypatch, c, k, relu):
     assert all(err[p] <= err[6] for p in PARTS_CFGS), err
 
 
+@pytest.mark.parametrize("implicit", ["0", "1"])
 @pytest.mark.parametrize("cfg", PARTS_CFGS)
-def test_parts_special_values(gpu, monkeypatch, cfg):
+def test_parts_special_values(gpu, monkeypatch, cfg, implicit):
     """Infinities, NaN, values next to the largest and the smallest floats
     give what the fp32 tile gives, and only where it does."""
+    monkeypatch.setenv("SPKV2_IMPLICIT_PAD", implicit)
     rng = np.random.default_rng(3)
     w = rng.standard_normal((40, 32, 3, 3)).astype(np.float32)
     w[5, 3, 1, 1], w[6, 4, 0, 0] = np.inf, np.nan
