@@ -44,6 +44,7 @@ enum ConvPath {
 struct GatherGeom {
     int C = 0, cstride = 0, KW = 1, tap_h = 0, tap_w = 0;
     bool kvec = false;
+    bool rows = false;  // k is contiguous (kvec or not), one pixel per image
     // implicit padding: the B source is the unpadded input (H x W, padded by
     // ph / pw at the top / left), every tap bounds-checked through the tap
     // table ktap (device, owned by the plan)

@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(256) conv_igemm_f32(IgemmArgs a) {
 #undef IGEMM_LOAD_B
 #undef IGEMM_STORE_B
 
-        igemm_epilogue<BM, BN, 32, TM, TN>(a, acc, mt, nt, wm, wn, lane, part, slice);
+        igemm_epilogue<BM, BN, 32, TM, TN, KVEC>(a, acc, mt, nt, wm, wn, lane, part, slice);
     }
 }
 
@@ -844,8 +844,10 @@ __global__ void __launch_bounds__(256) conv_thin_f32(IgemmArgs a) {
 
 // Sums split-K partials in slice order, then applies the epilogue.  Each
 // thread owns VEC consecutive columns of one row (VEC = 4 when the partial
-// columns start and end on multiples of 4: 16-byte loads).
-template <int VEC>
+// columns start and end on multiples of 4: 16-byte loads), or with ROWS (one
+// pixel per image, partials [slice][n][m]: igemm_epilogue) VEC consecutive
+// rows of one column.
+template <int VEC, bool ROWS>
 __global__ void __launch_bounds__(256) splitk_epilogue(const float *__restrict__ ws, int splitk, int M, int ld,
                                                        int OHW, const float *__restrict__ bias,
                                                        const float *__restrict__ res, float *__restrict__ y, int act,
@@ -857,17 +859,19 @@ __global__ void __launch_bounds__(256) splitk_epilogue(const float *__restrict__
     for (size_t gi = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; gi < groups;
          gi += static_cast<size_t>(gridDim.x) * 256) {
         const size_t idx = gi * VEC;
-        const int m = static_cast<int>(idx / ld);
-        const int n = h.ws_n0 + static_cast<int>(idx - static_cast<size_t>(m) * ld);
+        const int inner = ROWS ? M : ld;
+        const int outer = static_cast<int>(idx / inner), first = static_cast<int>(idx - static_cast<size_t>(outer) * inner);
+        const int m0 = ROWS ? first : outer;
+        const int n0 = h.ws_n0 + (ROWS ? outer : first);
         // bias and residual loads issued first: their latency overlaps the
         // partials'
-        const float bm = bias ? bias[m] : 0.0f;
-        float rv[VEC];
+        float bm[VEC], rv[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
-            const int img = (n + e) / OHW;
-            rv[e] = res ? res[static_cast<size_t>(img) * h.y_img_stride + static_cast<size_t>(m) * OHW +
-                              (n + e - img * OHW)]
+            const int m = m0 + (ROWS ? e : 0), n = n0 + (ROWS ? 0 : e);
+            const int img = n / OHW;
+            bm[e] = bias ? bias[m] : 0.0f;
+            rv[e] = res ? res[static_cast<size_t>(img) * h.y_img_stride + static_cast<size_t>(m) * OHW + (n - img * OHW)]
                         : 0.0f;
         }
         // up to 16 slices' loads in flight before the first add (one round
@@ -884,10 +888,11 @@ __global__ void __launch_bounds__(256) splitk_epilogue(const float *__restrict__
         }
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
+            const int m = m0 + (ROWS ? e : 0), n = n0 + (ROWS ? 0 : e);
             float o = alpha * v[e];
-            if (bias) o += bm;
-            const int img = (n + e) / OHW;
-            const int sp = n + e - img * OHW;
+            if (bias) o += bm[e];
+            const int img = n / OHW;
+            const int sp = n - img * OHW;
             const size_t yi = static_cast<size_t>(img) * h.y_img_stride + static_cast<size_t>(m) * h.y_cstride + sp;
             if (res) o += rv[e];
             o = apply_act(o, act);
@@ -1622,20 +1627,21 @@ static int launch_igemm(hipStream_t st, int cfg, const TileCounts &tc, const Con
     a.chk_dh = g.dh;
     a.chk_dw = g.dw;
     // 16-byte B loads need a 16-byte aligned source (a caller-bound input may not be)
-    const bool kvec = gg.kvec && (reinterpret_cast<uintptr_t>(xs) & 15) == 0;
+    // (those of conv_split_f32 do not: its rows may start anywhere)
+    const bool kvec = t.split_threads > 0 ? gg.rows && gg.C >= 4 : gg.kvec && (reinterpret_cast<uintptr_t>(xs) & 15) == 0;
+    a.sk_C = gg.C;
     (kvec ? t.kernel_kvec : gg.chk ? t.kernel_chk : t.kernel)<<<grid, dim3(cfg_threads(cfg)), 0, st>>>(a);
     if (int rc = launch_status("conv_igemm_f32")) return rc;
     if (tc.splitk > 1) {
         const size_t total = static_cast<size_t>(g.M) * a.ws_ld;
-        // four columns per thread where that still gives every CU a
-        // workgroup; small (batch-1) outputs take one column per thread, so
-        // the partial loads spread over more CUs
-        if (a.ws_ld % 4 == 0 && a.ws_n0 % 4 == 0 && total / 4 >= 256u * 256u)
-            hipLaunchKernelGGL(splitk_epilogue<4>, dim3(grid_for(total / 4, 256)), dim3(256), 0, st, ws, tc.splitk,
-                               g.M, a.ws_ld, a.OHW, bias, res, y, g.act, alpha, a);
-        else
-            hipLaunchKernelGGL(splitk_epilogue<1>, dim3(grid_for(total, 256)), dim3(256), 0, st, ws, tc.splitk, g.M,
-                               a.ws_ld, a.OHW, bias, res, y, g.act, alpha, a);
+        // four outputs per thread where that still gives every CU a
+        // workgroup; small (batch-1) outputs take one per thread, so the
+        // partial loads spread over more CUs
+        const bool quads = (kvec ? g.M % 4 == 0 : a.ws_ld % 4 == 0 && a.ws_n0 % 4 == 0) && total / 4 >= 256u * 256u;
+        const auto kernel = kvec ? (quads ? splitk_epilogue<4, true> : splitk_epilogue<1, true>)
+                                 : (quads ? splitk_epilogue<4, false> : splitk_epilogue<1, false>);
+        hipLaunchKernelGGL(kernel, dim3(grid_for(quads ? total / 4 : total, 256)), dim3(256), 0, st, ws, tc.splitk, g.M,
+                           a.ws_ld, a.OHW, bias, res, y, g.act, alpha, a);
         if (int rc = launch_status("splitk_epilogue")) return rc;
     }
     return 0;
@@ -2179,6 +2185,7 @@ int plan_igemm_gemm(hipStream_t st, const ConvGeom &g, const float *w_host, int 
     gs.key = shape_key(k_stride == 1 ? "gemm" : "gemm_ta", g, plan, gs.x_img_stride);
     gs.gather.C = g.C;  // one tap
     gs.gather.cstride = k_stride;
+    gs.gather.rows = k_stride == 1;
     gs.gather.kvec = k_stride == 1 && g.C % 4 == 0;  // A is [rows][K]: four k of a row are 16 contiguous bytes
     if (int rc = plan_tiles_and_weights(st, g, gs, w_host, plan)) return rc;
     plan->workspace = partial_bytes(plan);

@@ -141,12 +141,18 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
     constexpr int KG = BK / 8;           // 16-byte k groups per plane and column
     constexpr int KPT = BK * BN / NT;    // B elements per thread per k-tile
     constexpr int GPT = KPT / 8;         // k groups per thread
+    // B is a matrix of rows (a Gemm's A): eight lanes read the 32 k of a row,
+    // four each, where lane-per-column loads would touch a line per lane
+    constexpr bool ROWMAJOR = MODE == kModeKvec;
+    constexpr int RPP = NT / 8;          // rows per pass of the workgroup
+    constexpr int PAD = ROWMAJOR ? 4 : 0;  // keeps its 8-byte LDS writes off each other's banks
+    static_assert(BK == 32 && (!ROWMAJOR || BN % RPP == 0), "row-major pass");
     static_assert(TM >= 1 && TN >= 1 && KPT % 8 == 0 && BN >= 64 && NT % BN == 0, "tile shape");
 
     // [buffer][plane][k group][column] 16-byte pieces: a thread writes the
     // pieces of its column, a wave reads 32 columns of two groups, both
     // contiguous across lanes (no bank conflicts without padding)
-    __shared__ __attribute__((aligned(16))) uintx4 Bs[2][3][KG][BN];
+    __shared__ __attribute__((aligned(16))) uintx4 Bs[2][3][KG][BN + PAD];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -204,6 +210,18 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
         }
     }
 
+    // row-major B: this lane's first k of a tile, and its rows
+    const int K = a.sk_C;
+    const int rk = (tid & 7) * 4;
+    int rowoff[ROWMAJOR ? BN / RPP : 1];
+    if constexpr (ROWMAJOR) {
+#pragma unroll
+        for (int p = 0; p < BN / RPP; p++) {
+            const int n = nt * BN + (tid >> 3) + p * RPP;
+            rowoff[p] = n < a.Ntot ? n * a.x_img_stride * 4 : kOobOffset;
+        }
+    }
+
     // A: [m_tile][k_tile][32-row block][k step][part][lane] 16-byte pieces
     const bf16x8 *const wbase = reinterpret_cast<const bf16x8 *>(a.wp) +
                                 (static_cast<size_t>(mt) * a.k_tiles * (BM / 32) + wm * TM) * (Q * 3 * 64) + lane;
@@ -224,6 +242,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
     int ko[KPT];
     unsigned tap[MODE == kModeChk ? KPT : 1];
     auto load_ko = [&](int kt) __attribute__((always_inline)) {
+        if constexpr (ROWMAJOR) return;
 #pragma unroll
         for (int j = 0; j < KPT; j++) {
             ko[j] = a.koff[kt * BK + bgrp * KPT + j];
@@ -231,16 +250,20 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
         }
     };
     auto load_b = [&](int kt, float (&br)[KPT]) __attribute__((always_inline)) {
-        if constexpr (MODE == kModeKvec) {
+        if constexpr (ROWMAJOR) {
+            // the quad of the last tile that K cuts is read from K - 4 on
+            // and shifted into place when it is split (store_b)
+            const int k4 = min(kt * BK + rk, K - 4) * 4;
 #pragma unroll
-            for (int j = 0; j < KPT; j += 4) {
+            for (int p = 0; p < BN / RPP; p++) {
                 const floatx4 v =
-                    __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xrs, col, ko[j], 0));
-                br[j] = v[0];
-                br[j + 1] = v[1];
-                br[j + 2] = v[2];
-                br[j + 3] = v[3];
+                    __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(xrs, rowoff[p] + k4, 0, 0));
+                br[4 * p] = v[0];
+                br[4 * p + 1] = v[1];
+                br[4 * p + 2] = v[2];
+                br[4 * p + 3] = v[3];
             }
+            return;
         } else if constexpr (MODE == kModeChk) {
 #pragma unroll
             for (int j = 0; j < KPT; j++)
@@ -253,7 +276,36 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
         }
         load_ko(kt + 1);
     };
-    auto store_b = [&](int buf, const float (&br)[KPT]) __attribute__((always_inline)) {
+    auto store_b = [&](int kt, int buf, const float (&br)[KPT]) __attribute__((always_inline)) {
+        if constexpr (ROWMAJOR) {
+            float v[KPT];
+#pragma unroll
+            for (int j = 0; j < KPT; j++) v[j] = br[j];
+            if ((kt + 1) * BK > K) {
+                const int shift = kt * BK + rk - min(kt * BK + rk, K - 4);
+#pragma unroll
+                for (int p = 0; p < BN / RPP; p++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        float t = 0.0f;  // past K
+#pragma unroll
+                        for (int f = e; f < 4; f++) t = f == e + shift ? br[4 * p + f] : t;
+                        v[4 * p + e] = t;
+                    }
+            }
+#pragma unroll
+            for (int p = 0; p < BN / RPP; p++) {
+                unsigned h[2], m[2], l[2];
+                split_pair(v[4 * p], v[4 * p + 1], h[0], m[0], l[0]);
+                split_pair(v[4 * p + 2], v[4 * p + 3], h[1], m[1], l[1]);
+                uintx4 *at = &Bs[buf][0][rk / 8][(tid >> 3) + p * RPP];
+                const int q = rk / 4 & 1;
+                reinterpret_cast<uintx2 *>(at)[q] = uintx2{h[0], h[1]};
+                reinterpret_cast<uintx2 *>(at + KG * (BN + PAD))[q] = uintx2{m[0], m[1]};
+                reinterpret_cast<uintx2 *>(at + 2 * KG * (BN + PAD))[q] = uintx2{l[0], l[1]};
+            }
+            return;
+        }
 #pragma unroll
         for (int g = 0; g < GPT; g++) {
             uintx4 h, m, l;
@@ -316,7 +368,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
         load_b(kt + 2, bfree);
         load_a(kt + 1, an);
         __builtin_amdgcn_sched_barrier(0);
-        compute(buf, ac, [&]() __attribute__((always_inline)) { store_b(buf ^ 1, bnx); });
+        compute(buf, ac, [&]() __attribute__((always_inline)) { store_b(kt + 1, buf ^ 1, bnx); });
         __syncthreads();
     };
 
@@ -324,7 +376,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
     load_b(kt0, br0);
     load_b(kt0 + 1, br1);
     load_a(kt0, a0);
-    store_b(0, br0);
+    store_b(kt0, 0, br0);
     __syncthreads();
     int kt = kt0;
     // tiles past kt1 are loaded and ignored, which keeps the loop free of
@@ -370,7 +422,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
                         if (e == (i * TN + j) * 16 + r) acc[i][j][r] = v;
         }
     }
-    igemm_epilogue<BM, BN, 32, TM, TN>(a, acc, mt, nt, wm, wn, lane, part, slice);
+    igemm_epilogue<BM, BN, 32, TM, TN, ROWMAJOR>(a, acc, mt, nt, wm, wn, lane, part, slice);
 }
 
 int pack_split(hipStream_t st, const float *w, int M, int K, int BM, int BK, int m_tiles, int k_tiles, void *out) {

@@ -59,13 +59,35 @@ struct IgemmArgs {
 // k at a time, or bounds-checked taps of the unpadded input.
 constexpr int kModePlain = 0, kModeKvec = 1, kModeChk = 2;
 
+// Four consecutive outputs from v[r], `left` of which are inside the tensor,
+// at byte offset `off` (out of range past the last column): one 16-byte store
+// when they are all in or all out (quads).
+template <typename Block>
+__device__ __forceinline__ void store_rows(const Block &v, int r, __amdgpu_buffer_rsrc_t rs, int off, int left,
+                                           bool quads) {
+    if (quads) {
+        const uintx4 o = {__float_as_uint(v[r]), __float_as_uint(v[r + 1]), __float_as_uint(v[r + 2]),
+                          __float_as_uint(v[r + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(o, rs, left > 0 ? off : kOobOffset, 0, 0);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r + e]), rs, e < left ? off + 4 * e : kOobOffset, 0,
+                                                  0);
+    }
+}
+
 // Epilogue of one BM x BN tile held as TM x TN accumulator blocks of BS x BS
 // outputs per wave (wave wm, wn of the tile): split-K partials, or alpha,
 // bias, residual and activation in registers, then y and / or the handoff
 // target.  A lane holds one column of a block (lane % BS) and, of a 32x32
 // block, rows 8*(r/4) + 4*(lane/32) + (r%4) for r = 0..15, of a 16x16 block
 // rows 4*(lane/16) + r for r = 0..3.
-template <int BM, int BN, int BS, int TM, int TN, typename Block>
+// ROWS: one pixel per image (a Gemm), so that a lane's groups of four rows are
+// four consecutive outputs: 16-byte accesses where M is a multiple of 4, and
+// split-K partials ordered [slice][n][m].  (Dword stores M * 4 bytes apart
+// touched a line per lane.)
+template <int BM, int BN, int BS, int TM, int TN, bool ROWS, typename Block>
 __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (&acc)[TM][TN], int mt, int nt, int wm,
                                                int wn, int lane, bool part, int slice) {
     constexpr int NR = BS * BS / 64;
@@ -86,7 +108,22 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             const int n = nt * BN + (wn * TN + j) * BS + row;
-            obase[j] = n < a.Ntot ? (slice * a.M * a.ws_ld + n - a.ws_n0) * 4 : kOobOffset;
+            obase[j] = n >= a.Ntot ? kOobOffset
+                       : ROWS      ? (slice * a.ws_ld + n - a.ws_n0) * a.M * 4
+                                   : (slice * a.M * a.ws_ld + n - a.ws_n0) * 4;
+        }
+        if constexpr (ROWS) {
+            const bool quads = (a.M & 3) == 0;
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int q = 0; q < NR / 4; q++) {
+                        const int m = mrow[i] + 8 * q;
+                        store_rows(acc[i][j], 4 * q, wrs, obase[j] + m * 4, a.M - m, quads);
+                    }
+            return;
         }
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -143,6 +180,31 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
                                                           brs, (mrow[i] + 8 * (r >> 2) + (r & 3)) * 4, 0, 0));
 #pragma unroll
                 for (int j = 0; j < JG; j++) v[j] += bv;
+            }
+            if constexpr (ROWS) {
+                const bool quads = (a.M & 3) == 0;
+                if (a.res) {
+#pragma unroll
+                    for (int j = 0; j < JG; j++)
+#pragma unroll
+                        for (int r = 0; r < NR; r++) {
+                            const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
+                            v[j][r] += __builtin_bit_cast(
+                                float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           rrs, m < a.M ? obase[j0 + j] + m * 4 : kOobOffset, 0, 0));
+                        }
+                }
+#pragma unroll
+                for (int j = 0; j < JG; j++) {
+#pragma unroll
+                    for (int r = 0; r < NR; r++) v[j][r] = apply_act(v[j][r], a.act);
+#pragma unroll
+                    for (int q = 0; q < NR / 4; q++) {
+                        const int m = mrow[i] + 8 * q;
+                        store_rows(v[j], 4 * q, yrs, obase[j0 + j] + m * 4, a.M - m, quads);
+                    }
+                }
+                continue;
             }
             if (a.res) {
                 Block rv[JG];

@@ -94,15 +94,41 @@ def test_parts_hybrid_schedule(gpu, monkeypatch, cfg):
 
 @pytest.mark.parametrize("trans_a", [0, 1])
 @pytest.mark.parametrize("cfg", PARTS_CFGS)
-@pytest.mark.parametrize("rows,k,m", [(5, 64, 10), (33, 36, 129), (130, 100, 65)])
-def test_parts_gemm(gpu, monkeypatch, rows, k, m, cfg, trans_a):
-    _force(monkeypatch, cfg)
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("rows,k,m", [(5, 64, 10), (33, 36, 129), (130, 100, 64), (70, 37, 65), (65, 4, 33), (6, 3, 8),
+                                      (129, 135, 132)])
+def test_parts_gemm(gpu, monkeypatch, rows, k, m, cfg, split, trans_a):
+    _force(monkeypatch, cfg, split)
     g = models.single_gemm(rows, k, m, trans_a=trans_a)
     xs = rng_inputs(g)
     a = xs[0].astype(np.float64).T if trans_a else xs[0].astype(np.float64)
     b, c = (g.tensors[t].data.astype(np.float64) for t in g.nodes[0].inputs[1:3])
     got = run_gpu(write_spk(g, "mi355x"), xs)[0].reshape(rows, m)
     assert np.all(np.abs(got - (a @ b + c)) <= (k / 8 + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b) + np.abs(c)))
+
+
+@pytest.mark.parametrize("cfg", [6, *PARTS_CFGS])
+def test_gemm_rows_at_any_address(gpu, monkeypatch, cfg):
+    """A caller's input one float past an aligned address, NaN around it."""
+    from spinnv2_amd.runtime import DeviceBuffer, Model
+
+    _force(monkeypatch, cfg, 2)
+    rows, k, m = 67, 70, 36
+    g = models.single_gemm(rows, k, m)
+    x = rng_inputs(g)[0]
+    whole = np.full(x.size + 9, np.nan, np.float32)
+    whole[1:1 + x.size] = x.ravel()
+    with Model(write_spk(g, "mi355x")) as mdl:
+        buf = DeviceBuffer(whole.nbytes)
+        buf.upload(whole)
+        view = type("View", (), {"ptr": type(buf.ptr)(buf.ptr.value + 4), "nbytes": x.nbytes})
+        mdl.bind_input(0, view)
+        mdl.run()
+        got = mdl.get_output(0).reshape(rows, m)
+        buf.free()
+    a = x.astype(np.float64)
+    b, c = (g.tensors[t].data.astype(np.float64) for t in g.nodes[0].inputs[1:3])
+    assert np.all(np.abs(got - (a @ b + c)) <= (k / 2 + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b) + np.abs(c)))
 
 
 @pytest.mark.parametrize("relu", [False, True])
