@@ -26,24 +26,11 @@
 // loads 75; the fp32 tiles take 117 us.
 #define SPK_SPLIT_DEFINE
 #include "igemm_split.hpp"
+#include "parts.hpp"
 
 namespace spk::kern {
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// x = hi + mid + lo: each the nearest bf16 of what the ones before leave, so
-// the sum is x exactly (three 8-bit significands hold the 24 of a float).
-// Two elements at a time, packed low half first.
-__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
-    h = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x0, x1}, bf16x2));
-    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
-    m = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{r0, r1}, bf16x2));
-    const float s0 = r0 - __uint_as_float(m << 16), s1 = r1 - __uint_as_float(m & 0xffff0000u);
-    l = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{s0, s1}, bf16x2));
-}
 
 // BM x BK tiles [m_tiles][k_tiles], each [BM/32][BK/16][3 parts][64 lanes][8]
 // bf16: lane l of a 32x32x16 step holds row l & 31, k = 8 * (l >> 5) + 0..7 of
@@ -400,9 +387,9 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
             acc[i][j] += sml[i][j];
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const float v = __builtin_fabsf(acc[i][j][r]);
+                const float v = acc[i][j][r];
                 const int e = (i * TN + j) * 16 + r;
-                const bool odd = !(v < __builtin_inff()) || (v < 0x1p-90f && v != 0.0f);
+                const bool odd = parts_unfit(v);
                 (e < 64 ? odd0 : odd1) |= static_cast<unsigned long long>(odd) << (e & 63);
             }
         }

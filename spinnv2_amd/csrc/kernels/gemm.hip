@@ -17,6 +17,7 @@
 
 #include "conv.hpp"
 #include "kernels.hpp"
+#include "parts.hpp"
 
 namespace spk::kern {
 
@@ -204,6 +205,204 @@ __global__ void __launch_bounds__(256) matmul_mfma(MatmulArgs p) {
     }
 }
 
+// Batched MatMul on bf16 parts (parts.hpp, conv_split.hip): one BM x 64 tile
+// per workgroup, BK k at a time, both operands split on their way into LDS
+// (pieces of 8 k of one row or column), two tiles of loads in flight.
+//   BM = 32, BK = 64: waves 0 and 1 sum the two column halves over the first
+//   32 k of every tile, waves 2 and 3 over the others, and the two halves are
+//   added through LDS at the end.  For long k on few tiles (attention at small
+//   batches), a chain of K / 64 steps bound by their latency.
+//   BM = 64, BK = 32: four waves side by side, for the others.
+// TA / TB: the operand is stored transposed (A [K][M], B [N][K]), so that a
+// Transpose in front of it need not run.  Sixteen attention products at 20x20:
+// [400 x 32] x [32 x 400] 8.9 us behind its Transpose's 3 before, 8.9 alone
+// now, [64 x 400] x [400 x 400] 19 us behind a Transpose's 8.2, now 8.7; one
+// 2048^3 product 364 us on the fp32 tiles, now 143.
+constexpr int kPtN = 64, kPtPad = 2;
+
+// One operand's BK-k tile of R rows (columns of B) in registers: R * BK / 256
+// elements a thread, all loads in flight.  KCONT: k is contiguous, `ld` apart
+// by row (QUADS: K is a multiple of 4, so that a lane's four k are all in or all
+// out); otherwise rows are contiguous, `ld` apart by k.
+template <int R, int BK, bool KCONT, bool QUADS>
+struct PartTile {
+    static constexpr int N = R * BK / 256;
+    static constexpr int LPR = BK / 4;       // KCONT: lanes a row
+    static constexpr int RPP = 256 / LPR;    // KCONT: rows a pass
+    static_assert(R % RPP == 0 || !KCONT, "whole passes");
+    static_assert(N % 8 == 0, "whole pieces");
+    float v[N];
+
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int ld, int r0, int rows, int k0, int K, int tid) {
+        constexpr int kOob = 0x7fff0000;
+        if constexpr (KCONT) {
+            const int k = k0 + tid % LPR * 4;
+#pragma unroll
+            for (int p = 0; p < R / RPP; p++) {
+                const int r = r0 + tid / LPR + RPP * p;
+                const int off = r < rows ? (r * ld + k) * 4 : kOob;
+                if constexpr (QUADS) {
+                    const floatx4 q = __builtin_bit_cast(
+                        floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, k < K ? off : kOob, 0, 0));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[4 * p + e] = q[e];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        v[4 * p + e] = __builtin_bit_cast(
+                            float, __builtin_amdgcn_raw_buffer_load_b32(rs, k + e < K ? off + 4 * e : kOob, 0, 0));
+                }
+            }
+        } else {
+            const int r = r0 + tid % R, g = tid / R * N;
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const int k = k0 + g + j;
+                v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                     rs, r < rows && k < K ? (k * ld + r) * 4 : kOob, 0, 0));
+            }
+        }
+    }
+    // pieces [part][k group][row]
+    __device__ __forceinline__ void store(uintx4 (*lds)[BK / 8][R + kPtPad], int tid) const {
+        if constexpr (KCONT) {
+            const int g = tid % LPR >> 1, half = tid & 1;
+#pragma unroll
+            for (int p = 0; p < R / RPP; p++) {
+                unsigned h[2], m[2], l[2];
+                split_pair(v[4 * p], v[4 * p + 1], h[0], m[0], l[0]);
+                split_pair(v[4 * p + 2], v[4 * p + 3], h[1], m[1], l[1]);
+                const int r = tid / LPR + RPP * p;
+                reinterpret_cast<uintx2 *>(&lds[0][g][r])[half] = uintx2{h[0], h[1]};
+                reinterpret_cast<uintx2 *>(&lds[1][g][r])[half] = uintx2{m[0], m[1]};
+                reinterpret_cast<uintx2 *>(&lds[2][g][r])[half] = uintx2{l[0], l[1]};
+            }
+        } else {
+#pragma unroll
+            for (int g8 = 0; g8 < N / 8; g8++) {
+                uintx4 h, m, l;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    unsigned hv, mv, lv;
+                    split_pair(v[8 * g8 + 2 * e], v[8 * g8 + 2 * e + 1], hv, mv, lv);
+                    h[e] = hv;
+                    m[e] = mv;
+                    l[e] = lv;
+                }
+                const int g = tid / R * (N / 8) + g8, r = tid % R;
+                lds[0][g][r] = h;
+                lds[1][g][r] = m;
+                lds[2][g][r] = l;
+            }
+        }
+    }
+};
+
+template <int BM, bool TA, bool TB, bool QUADS>
+__global__ void __launch_bounds__(256) matmul_parts(MatmulArgs p) {
+    constexpr int BK = BM == 32 ? 64 : 32;
+    __shared__ __attribute__((aligned(16))) uintx4 As[2][3][BK / 8][BM + kPtPad];
+    __shared__ __attribute__((aligned(16))) uintx4 Bs[2][3][BK / 8][kPtN + kPtPad];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane & 31, half = lane >> 5;
+    const int wn = wave & 1;
+    const int wk = BM == 32 ? wave >> 1 : 0, wm = BM == 32 ? 0 : wave >> 1;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * kPtN;
+    size_t ab = 0, bb = 0;
+    matmul_batch(p, blockIdx.z, &ab, &bb);
+    const float *A = p.a + ab * p.M * p.K;
+    const float *B = p.b + bb * p.K * p.N;
+    float *Y = p.y + static_cast<size_t>(blockIdx.z) * p.M * p.N;
+    const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), static_cast<short>(0),
+                                                                         p.M * p.K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), static_cast<short>(0),
+                                                                         p.K * p.N * 4, 0x00020000);
+    PartTile<BM, BK, !TA, QUADS> a0, a1;
+    PartTile<kPtN, BK, TB, QUADS> b0, b1;
+    const int lda = TA ? p.M : p.K, ldb = TB ? p.K : p.N;
+    const int tiles = (p.K + BK - 1) / BK;
+
+    floatx16 acc, sml;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = sml[r] = 0.0f;
+    // tiles past the last load zeros without a memory access
+    auto load = [&](int t, PartTile<BM, BK, !TA, QUADS> &at, PartTile<kPtN, BK, TB, QUADS> &bt) __attribute__((always_inline)) {
+        at.load(ars, lda, m0, p.M, t * BK, p.K, tid);
+        bt.load(brs, ldb, n0, p.N, t * BK, p.K, tid);
+    };
+    auto step = [&](int t, int buf, const PartTile<BM, BK, !TA, QUADS> &an, const PartTile<kPtN, BK, TB, QUADS> &bn,
+                    PartTile<BM, BK, !TA, QUADS> &af, PartTile<kPtN, BK, TB, QUADS> &bf) __attribute__((always_inline)) {
+        load(t + 2, af, bf);
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int g = 4 * wk + 2 * q + half;
+            bf16x8 a[3], b[3];
+#pragma unroll
+            for (int s = 0; s < 3; s++) {
+                a[s] = __builtin_bit_cast(bf16x8, As[buf][s][g][wm * 32 + row]);
+                b[s] = __builtin_bit_cast(bf16x8, Bs[buf][s][g][wn * 32 + row]);
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], acc, 0, 0, 0);
+            sml = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], sml, 0, 0, 0);
+            sml = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], sml, 0, 0, 0);
+            sml = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], sml, 0, 0, 0);
+            sml = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], sml, 0, 0, 0);
+            sml = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], sml, 0, 0, 0);
+        }
+        an.store(As[buf ^ 1], tid);
+        bn.store(Bs[buf ^ 1], tid);
+        __syncthreads();
+    };
+    load(0, a0, b0);
+    load(1, a1, b1);
+    a0.store(As[0], tid);
+    b0.store(Bs[0], tid);
+    __syncthreads();
+    for (int t = 0; t < tiles; t += 2) {
+        step(t, 0, a1, b1, a0, b0);
+        if (t + 1 < tiles) step(t + 1, 1, a0, b0, a1, b1);
+    }
+    acc += sml;
+    if constexpr (BM == 32) {
+        // the second k half's sums, 16 floats a lane, through LDS
+        floatx4 *red = reinterpret_cast<floatx4 *>(&As[0][0][0][0]);
+        static_assert(sizeof(As) >= 2 * 64 * 16 * 4, "room for two waves' sums");
+        if (wk == 1) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                red[(wn * 4 + q) * 64 + lane] = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+        }
+        __syncthreads();
+        if (wk == 1) return;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const floatx4 v = red[(wn * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[4 * q + e] += v[e];
+        }
+    }
+    // accumulator layout: column lane & 31, rows 8*(r/4) + 4*(lane/32) + r%4
+    const int n = n0 + wn * 32 + row;
+    unsigned odd = 0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+        odd |= static_cast<unsigned>(parts_unfit(acc[r])) << r;
+        if (m < p.M && n < p.N) Y[static_cast<size_t>(m) * p.N + n] = acc[r];
+    }
+    if (n >= p.N) return;
+    for (; odd; odd &= odd - 1) {
+        const int r = __ffs(odd) - 1;
+        const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (m >= p.M) continue;
+        float s = 0.0f;
+        for (int k = 0; k < p.K; k++)
+            s = fmaf(A[TA ? static_cast<size_t>(k) * p.M + m : static_cast<size_t>(m) * p.K + k],
+                     B[TB ? static_cast<size_t>(n) * p.K + k : static_cast<size_t>(k) * p.N + n], s);
+        Y[static_cast<size_t>(m) * p.N + n] = s;
+    }
+}
+
 // Batched MatMul for grids too small to fill the GPU with 64x64 tiles (the
 // PSA attention products at batch 1): one 32x32 tile per workgroup, its k
 // range cut into four contiguous quarters (whole groups of 8 k), one per
@@ -370,10 +569,10 @@ int matmul_run(Spkv2Context *ctx, const Spkv2NodeRecord *node, void *) {
     if (M > 0x7fffffffULL || N > 0x7fffffffULL || K > 0x7fffffffULL) return SPKV2_E_UNSUPPORTED;
     const uint64_t mt = (M + kMmTile - 1) / kMmTile, nt = (N + kMmTile - 1) / kMmTile;
     if (mt > 65535 || batch > 65535 || nt > 0x7fffffffULL) return SPKV2_E_UNSUPPORTED;
-    // 64x64 tiles for fewer than half the CUs: 32x32 tiles with k split over
-    // the waves instead (measured on the PSA attention products: 14 tiles at
-    // batch 1 27 -> 15 us of node time; 224 tiles at batch 16 the 64x64
-    // kernel is faster);
+    // on the fp32 matrix cores: 64x64 tiles for fewer than half the CUs: 32x32
+    // tiles with k split over the waves instead (measured on the PSA attention
+    // products: 14 tiles at batch 1 27 -> 15 us of node time; 224 tiles at
+    // batch 16 the 64x64 kernel is faster);
     // SPKV2_MATMUL_KSPLIT=0 / 1 forces either
     const uint64_t mt32 = (M + 31) / 32, nt32 = (N + 31) / 32;
     bool ksplit = mt * nt * batch < 128 && mt32 <= 65535;
@@ -393,6 +592,44 @@ int matmul_run(Spkv2Context *ctx, const Spkv2NodeRecord *node, void *) {
         p.ashape[i] = static_cast<int>(ar->shape[i]);
         p.bshape[i] = static_cast<int>(br->shape[i]);
     }
+    bool trans[2] = {false, false};
+    for (int slot = 0; slot < 2; slot++) {
+        const size_t at = 2 * static_cast<size_t>(node->id) + slot;
+        if (at >= ctx->matmul_src.size() || !ctx->matmul_src[at] || !handoffs_live(ctx)) continue;
+        trans[slot] = true;
+        (slot ? p.b : p.a) = dptr<const float>(ctx, ctx->matmul_src[at] - 1);
+    }
+    // (the parts kernel's offsets into one matrix are 31-bit)
+    const uint64_t limit = 0x7fff0000ULL / 4;
+    // 32 rows and k over the waves where k is long and the 64-row tiles would
+    // leave CUs idle (one 512^3 product, 64 tiles: 12.0 us against 13.7; eight
+    // of them, 512 tiles: 33 against 22); few tiles without a Transpose to
+    // save stay on the fp32 tiles, k split, whose loads go straight to
+    // registers (four 128^3 products: 3.6 us against 5.5)
+    const uint64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64) * batch;
+    const bool small = K > 64 && tiles64 < 256;
+    const int bm = small ? 32 : 64;
+    const uint64_t mt_pt = (M + bm - 1) / bm, nt_pt = (N + kPtN - 1) / kPtN;
+    const bool parts_fit = M * K < limit && K * N < limit && mt_pt <= 65535;
+    const bool reads_transposed = node->id < ctx->matmul_parts.size() && ctx->matmul_parts[node->id];
+    const bool parts = (tiles64 >= 64 || reads_transposed) && !getenv("SPKV2_MATMUL_KSPLIT");
+    if (parts_fit && (parts || trans[0] || trans[1])) {
+        set_kernel_name(ctx, node, "matmul_parts<" + std::to_string(bm) + "x64" + (trans[0] ? ",ta" : "") +
+                                       (trans[1] ? ",tb" : "") + ">");
+        using Kernel = void (*)(MatmulArgs);
+#define PARTS_TILE(BM, Q)                                                                    \
+    {{matmul_parts<BM, false, false, Q>, matmul_parts<BM, false, true, Q>},                  \
+     {matmul_parts<BM, true, false, Q>, matmul_parts<BM, true, true, Q>}}
+        const Kernel kernels[2][2][2][2] = {{PARTS_TILE(64, false), PARTS_TILE(32, false)},
+                                            {PARTS_TILE(64, true), PARTS_TILE(32, true)}};
+#undef PARTS_TILE
+        hipLaunchKernelGGL(kernels[K % 4 == 0][small][trans[0]][trans[1]],
+                           dim3(static_cast<unsigned>(nt_pt), static_cast<unsigned>(mt_pt),
+                                static_cast<unsigned>(batch)),
+                           dim3(256), 0, ctx->stream, p);
+        return launch_status("matmul");
+    }
+    if (trans[0] || trans[1]) return SPKV2_E_UNSUPPORTED;  // not set up that way
     if (ksplit) {
         set_kernel_name(ctx, node, "matmul_ksplit_f32<32x32>");
         hipLaunchKernelGGL(matmul_ksplit, dim3(static_cast<unsigned>(nt32), static_cast<unsigned>(mt32),

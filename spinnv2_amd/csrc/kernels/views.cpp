@@ -26,6 +26,7 @@
 // ever overwritten there.  Like the other handoffs the views are in force
 // only while handoffs_live(): otherwise every node reads and writes its own
 // tensors, as the reference does.  SPKV2_CONCAT_VIEWS=0 turns them off.
+#include <algorithm>
 #include <cstdlib>
 #include <map>
 #include <utility>
@@ -273,14 +274,63 @@ void setup_head_views(Spkv2Context *ctx, const Uses &u) {
 
 }  // namespace
 
+// A MatMul operand that a Transpose of the last two axes made, for that
+// MatMul alone: the product reads the Transpose's input as it lies and the
+// Transpose does not run.  That input's place in the arena is free for other
+// tensors once the Transpose is past, so the tensor gets a buffer of its own
+// (only an activation whose one reader is the Transpose and that no shape-only
+// node aliases).
+int setup_matmul_operands(Spkv2Context *ctx, const Uses &u, bool views) {
+    for (uint32_t id = 0; id < ctx->header.num_nodes; id++) {
+        const Spkv2NodeRecord *n = &ctx->node_records[id];
+        if (n->op_type != SPKV2_OP_MATMUL || !builtin_runs(ctx, id) || n->input_count < 2) continue;
+        for (int slot = 0; slot < 2; slot++) {
+            const uint32_t t = n->inputs[slot];
+            const int pid = u.producer[t];
+            if (pid < 0 || u.readers[t].size() != 1 || u.graph_io[t] || ctx->views[t].base) continue;
+            const Spkv2NodeRecord *p = &ctx->node_records[pid];
+            if (p->op_type != SPKV2_OP_TRANSPOSE || !builtin_runs(ctx, p->id) || p->output_count != 1) continue;
+            Spkv2AttrRecord attr;
+            if (spkv2_ctx_get_attr(ctx, p, &attr) != 0) continue;
+            const uint32_t x = p->inputs[0];
+            const Spkv2TensorRecord *xr = rec(ctx, x), *tr = rec(ctx, t);
+            const int rank = xr->rank;
+            bool swaps = rank >= 2 && tr->rank == rank && attr.extra_count == rank && attr.extra[rank - 1] == rank - 2 &&
+                         attr.extra[rank - 2] == rank - 1;
+            for (int d = 0; d + 2 < rank && swaps; d++) swaps = attr.extra[d] == d;
+            const uint64_t matrix = static_cast<uint64_t>(rank >= 2 ? xr->shape[rank - 1] : 0) * xr->shape[rank >= 2 ? rank - 2 : 0];
+            const Spkv2TensorRecord *o = rec(ctx, n->inputs[1 - slot]);
+            const uint64_t other = o->rank >= 2 ? static_cast<uint64_t>(o->shape[o->rank - 1]) * o->shape[o->rank - 2] : ~0ull;
+            if (std::max(matrix, other) >= 0x7fff0000ull / 4) continue;  // matmul_parts' offsets
+            if (!swaps || !movable_rank(ctx, u, x, rank) || u.readers[x].size() != 1 || ctx->moved[x]) continue;
+            const int xp = u.producer[x];
+            if (xp < 0 || !builtin_runs(ctx, static_cast<uint32_t>(xp))) continue;
+            const uint16_t op = ctx->node_records[xp].op_type;
+            if (op != SPKV2_OP_SPLIT && op != SPKV2_OP_SOFTMAX && op != SPKV2_OP_MATMUL && op != SPKV2_OP_ADD &&
+                op != SPKV2_OP_MUL)
+                continue;
+            ctx->matmul_parts[id] = 1;
+            if (!views) continue;
+            void *buf = nullptr;
+            if (int rc = hip_check(hipMalloc(&buf, xr->size_bytes), "hipMalloc MatMul operand")) return rc;
+            ctx->view_buffers.push_back(buf);
+            ctx->moved[x] = static_cast<uint8_t *>(buf);
+            ctx->tensors[x].data = ctx->moved[x];
+            ctx->matmul_src[2 * id + slot] = x + 1;
+            ctx->view_elide[p->id] = 1;
+        }
+    }
+    return 0;
+}
+
 int setup_concat_views(Spkv2Context *ctx) {
     const uint32_t nt = ctx->header.num_tensors, nn = ctx->header.num_nodes;
     ctx->views.assign(nt, Spkv2TensorView{});
     ctx->view_split.assign(nn, 0);
     ctx->view_elide.assign(nn, 0);
-    if (ctx->protection_count > 0) return 0;  // protected packages keep every tensor where the reference has it
-    if (const char *e = getenv("SPKV2_CONCAT_VIEWS"))
-        if (e[0] == '0') return 0;
+    ctx->moved.assign(nt, nullptr);
+    ctx->matmul_src.assign(2 * static_cast<size_t>(nn), 0);
+    ctx->matmul_parts.assign(nn, 0);
     Uses u;
     u.producer.assign(nt, -1);
     u.readers.assign(nt, {});
@@ -294,6 +344,9 @@ int setup_concat_views(Spkv2Context *ctx) {
         for (uint16_t q = 0; q < n->input_count; q++)
             if (n->inputs[q] < nt) u.readers[n->inputs[q]].push_back({i, q});
     }
+    // protected packages keep every tensor where the reference has it
+    const char *env = getenv("SPKV2_CONCAT_VIEWS");
+    if (ctx->protection_count > 0 || (env && env[0] == '0')) return setup_matmul_operands(ctx, u, false);
     for (uint32_t id = 0; id < nn; id++) {
         const Spkv2NodeRecord *k = &ctx->node_records[id];
         if (k->op_type != SPKV2_OP_CONCAT || !builtin_runs(ctx, id) || k->output_count != 1) continue;
@@ -342,7 +395,7 @@ int setup_concat_views(Spkv2Context *ctx) {
         for (uint32_t s : pl.splits) ctx->view_split[s] = 1;
     }
     setup_head_views(ctx, u);
-    return 0;
+    return setup_matmul_operands(ctx, u, true);
 }
 
 }  // namespace spk::kern

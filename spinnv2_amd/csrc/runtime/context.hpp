@@ -146,6 +146,15 @@ struct Spkv2Context {
     std::vector<uint8_t> view_split;
     std::vector<uint8_t> view_elide;  // nodes whose output the views already hold: nothing to run
     std::vector<void *> view_buffers;
+    // Tensors moved out of the arena into a buffer of their own (null: none),
+    // and per MatMul operand (2 * node + slot) the tensor, plus one, that it
+    // reads transposed while the handoffs are in force (0: its own input)
+    std::vector<uint8_t *> moved;
+    std::vector<uint32_t> matmul_src;
+    // MatMul nodes with such an operand: they run on the kernel that can read
+    // it so whether or not the handoffs are in force, so that the results are
+    // the same bits
+    std::vector<uint8_t> matmul_parts;
     // int8 activation tensors (per tensor id; buf null for every other
     // tensor) and the nodes that read or write one
     std::vector<Spkv2Q8Tensor> q8;

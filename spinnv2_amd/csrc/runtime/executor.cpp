@@ -408,7 +408,7 @@ extern "C" int spkv2_prepare_with_scratch(Spkv2Context *ctx, void *arena, size_t
             ctx->tensors[i].data = nullptr;
         } else {
             if (r->data_offset + r->size_bytes > required) return -4;
-            ctx->tensors[i].data = ctx->arena + r->data_offset;
+            ctx->tensors[i].data = i < ctx->moved.size() && ctx->moved[i] ? ctx->moved[i] : ctx->arena + r->data_offset;
         }
     }
     ctx->binding_epoch++;

@@ -1,0 +1,101 @@
+"""Batched MatMul on bf16 parts, and MatMul operands read transposed in place
+of a Transpose node, against 64-bit products.
+
+|error| <= (K / 8 + 16) * 2^-24 * sum |a b|, as for the convolutions on parts.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from spinnv2_amd.runtime import Model
+from spinnv2_amd.spk import models, write_spk
+from spinnv2_amd.spk.graph import Graph
+
+from .helpers import rng_inputs, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, a, b):
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    want, size = a @ b, np.abs(a) @ np.abs(b)
+    assert np.all(np.abs(got.reshape(want.shape) - want) <= (a.shape[-1] / 8 + 16) * 2.0 ** -24 * size)
+
+
+# tiles' edges and remainders in M, N and K, on 64- and 32-row tiles
+@pytest.mark.parametrize("batch,m,n,k", [(70, 1, 1, 1), (64, 64, 64, 32), (16, 65, 127, 33), (70, 33, 66, 70),
+                                         (9, 129, 200, 31), (64, 31, 63, 130), (3, 400, 257, 101), (80, 5, 7, 64)])
+def test_matmul_parts(gpu, batch, m, n, k):
+    g = models.matmul_op([batch, m, k], [batch, k, n])
+    xs = rng_inputs(g)
+    with Model(write_spk(g, "mi355x")) as mdl:
+        got = mdl(*xs)
+        assert "matmul_parts" in mdl.kernel_name(0)
+    _close(got, *xs)
+
+
+@pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("batch,m,n,k", [(2, 20, 33, 12), (6, 64, 65, 130), (1, 100, 40, 67), (70, 64, 64, 32)])
+def test_transposed_operands(gpu, monkeypatch, batch, m, n, k, ta, tb):
+    """Transposes feeding only the MatMul are not run; with the views off they
+    are, and the results are the same bits."""
+    g = Graph("mm")
+    a = g.input("a", [batch, k, m] if ta else [batch, m, k])
+    b = g.input("b", [batch, n, k] if tb else [batch, k, n])
+    ga, gb = g.add(a, a), g.add(b, b)
+    ma = g.transpose(ga, [0, 2, 1]) if ta else ga
+    mb = g.transpose(gb, [0, 2, 1]) if tb else gb
+    g.mark_output(g.add(g.matmul(ma, mb), g.weight("zero", np.zeros(1, np.float32))))
+    xs = rng_inputs(g)
+    blob = write_spk(g, "mi355x")
+    with Model(blob) as mdl:
+        got = [mdl(*xs), mdl(*xs)]
+        names = [mdl.kernel_name(i) for i in range(len(g.nodes))]
+    assert sum("transpose_elided" in s for s in names) == ta + tb, names
+    assert any("matmul_parts" in s and (",ta" in s) == ta and (",tb" in s) == tb for s in names), names
+    np.testing.assert_array_equal(got[0], got[1])
+    xa, xb = (np.swapaxes(x, 1, 2) if t else x for x, t in zip(xs, (ta, tb)))
+    _close(got[0], 2 * xa, 2 * xb)
+    monkeypatch.setenv("SPKV2_CONCAT_VIEWS", "0")
+    with Model(blob) as mdl:
+        plain = mdl(*xs)
+        pnames = [mdl.kernel_name(i) for i in range(len(g.nodes))]
+    assert not any("elided" in s for s in pnames), pnames
+    np.testing.assert_array_equal(plain, got[0])
+
+
+def test_transposed_operand_with_a_fault_armed(gpu):
+    """With a fault event armed (here on a node's later invocation, so that
+    nothing flips) every node runs on its own tensors."""
+    g = Graph("mm")
+    a, b = g.input("a", [4, 40, 24]), g.input("b", [4, 40, 30])
+    s = g.softmax(a, -1)
+    g.mark_output(g.matmul(g.transpose(s, [0, 2, 1]), b))
+    xs = rng_inputs(g)
+    with Model(write_spk(g, "mi355x")) as mdl:
+        one = mdl(*xs)
+        assert mdl.set_fault_event({"node_id": 0, "tensor_id": g.nodes[0].outputs[0], "element_index": 0,
+                                    "bit_index": 1, "invocation_index": 9, "enabled": 1}) == 0
+        for i, x in enumerate(xs):
+            mdl.set_input(i, x)
+        mdl.run()
+        two = mdl.get_output(0)
+        assert not any("elided" in mdl.kernel_name(i) for i in range(len(g.nodes)))
+    np.testing.assert_array_equal(two, one)
+
+
+def test_matmul_special_values(gpu, monkeypatch):
+    g = models.matmul_op([64, 40, 70], [64, 70, 50])
+    xs = rng_inputs(g)
+    xs[0][0, 1, 2], xs[0][1, 3, 4], xs[1][2, 5, 6] = np.inf, np.nan, np.float32(3.4e38)
+    xs[0][3] *= 1e-36
+    got = run_gpu(write_spk(g, "mi355x"), xs)[0].reshape(64, 40, 50)
+    monkeypatch.setenv("SPKV2_MATMUL_KSPLIT", "0")
+    want = run_gpu(write_spk(g, "mi355x"), xs)[0].reshape(64, 40, 50)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fin = np.isfinite(want)
+    np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-4)
+    np.testing.assert_allclose(got[3], want[3], rtol=1e-4, atol=1e-40)
