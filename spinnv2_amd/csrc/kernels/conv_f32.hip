@@ -2291,12 +2291,15 @@ static int run_igemm_impl(Spkv2Context *ctx, const ConvPlan *p, const float *x, 
 // batch 16: 170 against 124 us with its copy), so they keep the copy; so
 // do the skinny kernel (it reads a padded input) and inputs 16384 or more
 // rows or columns tall (the tap table packs a tap into 16 bits).  The tiles
-// on bf16 parts check a tap with one and and one compare (tap_mask), and take
-// the checks with 128 rows, which share an element's check, always (the 14x14
-// 3x3 layer, 256 channels: batch 64 110 us with the copy, 109 without, batch 8
-// 33.4 and 31.1, 72 to 100 channels at 75x57 stride 2 29.9 and 24.4), with
-// fewer rows while the copy costs more than about 3% of the layer: below 6
-// GFLOP (64 rows, batch 64: 137 and 141 us; batch 8: 36.9 and 33.9).
+// on bf16 parts check a tap with one and and one compare (tap_mask): per
+// million elements gathered that is about 0.1 us, twice that with 32 rows, and
+// a copy costs about 3 us and 0.17 us per MB read and written, so they take
+// the checks where those come out cheaper.  With the copy and without, in us:
+// 14x14, 256 channels, 128 rows, batch 64 110 and 104; 64 channels at 80x80,
+// 64 rows, batch 16 74 and 67; 72 to 100 channels at 75x57, stride 2 29.6 and
+// 23.6; on the other side 256 channels at 56x56, 128 rows, batch 16 330 and
+// 341; 14x14, 64 rows, batch 64 133 and 141; 7x7 taps over 240 channels at
+// 30x201, 32 rows 106 and 118.
 // SPKV2_IMPLICIT_PAD=0 keeps the copy everywhere, =1 takes the checks
 // wherever they apply.
 static int use_implicit_padding(ConvPlan *plan) {
@@ -2307,10 +2310,14 @@ static int use_implicit_padding(ConvPlan *plan) {
     if (e && e[0] == '0') return 0;
     const bool parts = kCfgs[plan->cfg].split_threads > 0;
     if (parts && (g.KH > 15 || g.KW > 15)) return 0;  // its tap table has 15 bits a side
-    const double gflop = 2e-9 * static_cast<double>(g.y_elems) * g.C * g.KH * g.KW;
-    if (!(e && e[0] == '1') && g.C * g.KH * g.KW > 160 && !(parts && (plan->BM >= 128 || gflop < 6.0))) return 0;
     const int BK = plan->BK;
     const int K = g.C * g.KH * g.KW;
+    if (!(e && e[0] == '1') && K > 160) {
+        if (!parts) return 0;
+        const double gathered = 1e-6 * K * g.N * g.OH * g.OW * ((g.M + plan->BM - 1) / plan->BM);
+        const double copied = 4e-6 * g.N * g.C * (static_cast<double>(g.H) * g.W + static_cast<double>(plan->Hp) * plan->Wp);
+        if ((plan->BM < 64 ? 0.2 : 0.1) * gathered > 3.0 + 0.17 * copied) return 0;
+    }
     const size_t entries = static_cast<size_t>(plan->Kpad) + 3 * BK;  // as build_koff: three tiles past Kpad
     std::vector<int> koff(entries, kOobOffset), ktap(entries, parts ? -1 : 0x7fff7fff);
     for (int k = 0; k < K; k++) {
