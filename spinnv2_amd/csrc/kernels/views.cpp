@@ -323,6 +323,43 @@ int setup_matmul_operands(Spkv2Context *ctx, const Uses &u, bool views) {
     return 0;
 }
 
+// GatherElements indices that a Tile made, for that node alone: it reads the
+// Tile's input and the Tile does not run.  The input's place in the arena may
+// be given to another tensor once the Tile is past, so no node up to the
+// GatherElements may write there (in place of a buffer of its own: it is
+// often the output of a shape-only node, which shares its input's place).
+static void setup_tiled_indices(Spkv2Context *ctx, const Uses &u) {
+    for (uint32_t id = 0; id < ctx->header.num_nodes; id++) {
+        const Spkv2NodeRecord *n = &ctx->node_records[id];
+        if (n->op_type != SPKV2_OP_GATHERELEMENTS || !builtin_runs(ctx, id) || n->input_count < 2) continue;
+        const uint32_t t = n->inputs[1];
+        const int pid = u.producer[t];
+        if (pid < 0 || static_cast<uint32_t>(pid) >= id || u.readers[t].size() != 1 || u.graph_io[t] ||
+            ctx->views[t].base)
+            continue;
+        const Spkv2NodeRecord *p = &ctx->node_records[pid];
+        if (p->op_type != SPKV2_OP_TILE || !builtin_runs(ctx, p->id) || p->output_count != 1) continue;
+        const uint32_t x = p->inputs[0];
+        const Spkv2TensorRecord *xr = rec(ctx, x), *tr = rec(ctx, t);
+        if (xr->rank != tr->rank || !movable_rank(ctx, u, x, xr->rank) || ctx->moved[x]) continue;
+        const int xp = u.producer[x];
+        if (xp < 0 || ctx->view_elide[xp]) continue;  // x is written
+        const uint64_t x0 = xr->data_offset, x1 = x0 + xr->size_bytes;
+        bool kept = true;
+        for (uint32_t between = static_cast<uint32_t>(pid) + 1; between <= id && kept; between++) {
+            const Spkv2NodeRecord *b = &ctx->node_records[between];
+            for (uint16_t o = 0; o < b->output_count; o++) {
+                const Spkv2TensorRecord *w = rec(ctx, b->outputs[o]);
+                const uint64_t w0 = w->data_offset, w1 = w0 + w->size_bytes;
+                if (w->memory_class == SPKV2_MEMORY_ACTIVATION_ARENA && w0 < x1 && x0 < w1) kept = false;
+            }
+        }
+        if (!kept) continue;
+        ctx->gather_src[id] = x + 1;
+        ctx->view_elide[p->id] = 1;
+    }
+}
+
 int setup_concat_views(Spkv2Context *ctx) {
     const uint32_t nt = ctx->header.num_tensors, nn = ctx->header.num_nodes;
     ctx->views.assign(nt, Spkv2TensorView{});
@@ -331,6 +368,7 @@ int setup_concat_views(Spkv2Context *ctx) {
     ctx->moved.assign(nt, nullptr);
     ctx->matmul_src.assign(2 * static_cast<size_t>(nn), 0);
     ctx->matmul_parts.assign(nn, 0);
+    ctx->gather_src.assign(nn, 0);
     Uses u;
     u.producer.assign(nt, -1);
     u.readers.assign(nt, {});
@@ -395,6 +433,7 @@ int setup_concat_views(Spkv2Context *ctx) {
         for (uint32_t s : pl.splits) ctx->view_split[s] = 1;
     }
     setup_head_views(ctx, u);
+    setup_tiled_indices(ctx, u);
     return setup_matmul_operands(ctx, u, true);
 }
 

@@ -155,6 +155,9 @@ struct Spkv2Context {
     // it so whether or not the handoffs are in force, so that the results are
     // the same bits
     std::vector<uint8_t> matmul_parts;
+    // Per GatherElements node the tensor, plus one, whose Tile are its indices
+    // while the handoffs are in force (0: its own input)
+    std::vector<uint32_t> gather_src;
     // int8 activation tensors (per tensor id; buf null for every other
     // tensor) and the nodes that read or write one
     std::vector<Spkv2Q8Tensor> q8;
