@@ -811,7 +811,7 @@ def main() -> None:
                      "traffic_basis": "HBM bytes of all conv launches of one step (rocprofv3 FETCH_SIZE + "
                                       "WRITE_SIZE, copy-kernel scaled; profiles/)" if traffic else None,
                      "algorithmic_bytes": conv_alg_bytes,
-                     "kernel": "conv_igemm_f32 (all conv nodes)"},
+                     "kernel": "conv_split_f32 / conv_igemm_f32 (all conv nodes)"},
         "cpu_baseline": base,
         "cpu_baseline_simd": base_simd,
         "int8": int8,

@@ -21,6 +21,9 @@ int pack_split(hipStream_t st, const float *w, int M, int K, int BM, int BK, int
 // layers of at most 64 outputs and for few columns (56x56 3x3 at 64 channels:
 // 100 us against 164), and run 4 to 10% faster held to 128 registers; 32
 // rows for the thinnest layers.
+// Larger tiles lose what they save in loads and splits to fewer waves a CU:
+// 256x64 with eight waves 106 us against 108 on the 3x3 layer but 72 against
+// 62 on the 1x1 expand, 128x128 with 256 registers 218 and 92.
 #define SPK_SPLIT_TILES(T) T(128, 64, 32, 4, 1, 1, 1.25) T(64, 64, 32, 2, 2, 4, 1.1) T(32, 128, 32, 1, 4, 1, 0.9)
 
 #define SPK_SPLIT_EXTERN(BM, BN, BK, WM, WN, WPE, EFF)                                                \
