@@ -225,18 +225,24 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
                 for (int p = 0; p < 3; p++) ax[i][q][p] = src[((i * Q + q) * 3 + p) * 64];
     };
     // The k offsets are read one tile ahead of the loads that use them (the
-    // table has three tiles of out-of-range entries past K).
-    int ko[KPT];
-    unsigned tap[MODE == kModeChk ? KPT : 1];
-    auto load_ko = [&](int kt) __attribute__((always_inline)) {
+    // table has three tiles of out-of-range entries past K), in two sets taken
+    // in turn: a scalar load in flight makes every wait for LDS wait for it
+    // too, so it is issued ahead of the step's vector loads, which cover it
+    // (72 to 100 channels, stride 2, at 75x57, batch 5 33.2 -> 30.8 us; it also
+    // freed registers, and the checked 128- and 32-row tiles a third wave).
+    struct Offsets {
+        int ko[KPT];
+        unsigned tap[MODE == kModeChk ? KPT : 1];
+    } o0, o1;
+    auto load_ko = [&](int kt, Offsets &o) __attribute__((always_inline)) {
         if constexpr (ROWMAJOR) return;
 #pragma unroll
         for (int j = 0; j < KPT; j++) {
-            ko[j] = a.koff[kt * BK + bgrp * KPT + j];
-            if constexpr (MODE == kModeChk) tap[j] = static_cast<unsigned>(a.ktap[kt * BK + bgrp * KPT + j]);
+            o.ko[j] = a.koff[kt * BK + bgrp * KPT + j];
+            if constexpr (MODE == kModeChk) o.tap[j] = static_cast<unsigned>(a.ktap[kt * BK + bgrp * KPT + j]);
         }
     };
-    auto load_b = [&](int kt, float (&br)[KPT]) __attribute__((always_inline)) {
+    auto load_b = [&](int kt, float (&br)[KPT], const Offsets &o) __attribute__((always_inline)) {
         if constexpr (ROWMAJOR) {
             // the quad of the last tile that K cuts is read from K - 4 on
             // and shifted into place when it is split (store_b)
@@ -255,13 +261,12 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
 #pragma unroll
             for (int j = 0; j < KPT; j++)
                 br[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                      xrs, (valid & tap[j]) == tap[j] ? col : kOobOffset, ko[j], 0));
+                                                      xrs, (valid & o.tap[j]) == o.tap[j] ? col : kOobOffset, o.ko[j], 0));
         } else {
 #pragma unroll
             for (int j = 0; j < KPT; j++)
-                br[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, col, ko[j], 0));
+                br[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, col, o.ko[j], 0));
         }
-        load_ko(kt + 1);
     };
     auto store_b = [&](int kt, int buf, const float (&br)[KPT]) __attribute__((always_inline)) {
         if constexpr (ROWMAJOR) {
@@ -334,11 +339,17 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
     };
     // The five products of 2^-8 and below keep a sum of their own: added one
     // by one to the large one each would round at its size.
-    auto compute = [&](int buf, const bf16x8 (&ac)[TM][Q][3], auto &&between) __attribute__((always_inline)) {
+    auto compute = [&](int buf, const bf16x8 (&ac)[TM][Q][3], const bf16x8 (&first)[TN],
+                       auto &&between) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             bf16x8 bh[TN], bm[TN], bl[TN];
-            frag_b(buf, q, 0, bh);
+            if (q == 0) {
+#pragma unroll
+                for (int j = 0; j < TN; j++) bh[j] = first[j];
+            } else {
+                frag_b(buf, q, 0, bh);
+            }
             frag_b(buf, q, 1, bm);
             frag_b(buf, q, 2, bl);
             mma(ac, q, 0, bh, acc);
@@ -351,17 +362,23 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
         }
     };
     auto step = [&](int kt, int buf, const bf16x8 (&ac)[TM][Q][3], bf16x8 (&an)[TM][Q][3], const float (&bnx)[KPT],
-                    float (&bfree)[KPT]) __attribute__((always_inline)) {
-        load_b(kt + 2, bfree);
+                    float (&bfree)[KPT], const Offsets &oc, Offsets &on) __attribute__((always_inline)) {
+        bf16x8 first[TN];
+        load_ko(kt + 3, on);
+        frag_b(buf, 0, 0, first);
+        __builtin_amdgcn_sched_barrier(0);
+        load_b(kt + 2, bfree, oc);
         load_a(kt + 1, an);
         __builtin_amdgcn_sched_barrier(0);
-        compute(buf, ac, [&]() __attribute__((always_inline)) { store_b(kt + 1, buf ^ 1, bnx); });
+        compute(buf, ac, first, [&]() __attribute__((always_inline)) { store_b(kt + 1, buf ^ 1, bnx); });
         __syncthreads();
     };
 
-    load_ko(kt0);
-    load_b(kt0, br0);
-    load_b(kt0 + 1, br1);
+    load_ko(kt0, o0);
+    load_ko(kt0 + 1, o1);
+    load_b(kt0, br0, o0);
+    load_b(kt0 + 1, br1, o1);
+    load_ko(kt0 + 2, o0);
     load_a(kt0, a0);
     store_b(kt0, 0, br0);
     __syncthreads();
@@ -369,10 +386,14 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
     // tiles past kt1 are loaded and ignored, which keeps the loop free of
     // data-dependent branches
     for (; kt + 1 < kt1; kt += 2) {
-        step(kt, 0, a0, a1, br1, br0);
-        step(kt + 1, 1, a1, a0, br0, br1);
+        step(kt, 0, a0, a1, br1, br0, o0, o1);
+        step(kt + 1, 1, a1, a0, br0, br1, o1, o0);
     }
-    if (kt < kt1) compute(0, a0, []() {});
+    if (kt < kt1) {
+        bf16x8 first[TN];
+        frag_b(0, 0, 0, first);
+        compute(0, a0, first, []() {});
+    }
 
     // An infinite input or product has parts of both signs, whose sum is not
     // what a float32 sum gives, and the parts of values near the smallest
