@@ -325,9 +325,11 @@ int setup_matmul_operands(Spkv2Context *ctx, const Uses &u, bool views) {
 
 // GatherElements indices that a Tile made, for that node alone: it reads the
 // Tile's input and the Tile does not run.  The input's place in the arena may
-// be given to another tensor once the Tile is past, so no node up to the
-// GatherElements may write there (in place of a buffer of its own: it is
-// often the output of a shape-only node, which shares its input's place).
+// be given to another tensor once the Tile is past, so no node up to and
+// including the GatherElements may write there (in place of a buffer of its
+// own: it is often the output of a shape-only node, which shares its input's
+// place).  Graph outputs lie in the arena too unless they are external; one
+// that the caller binds elsewhere still counts, since it may be bound later.
 static void setup_tiled_indices(Spkv2Context *ctx, const Uses &u) {
     for (uint32_t id = 0; id < ctx->header.num_nodes; id++) {
         const Spkv2NodeRecord *n = &ctx->node_records[id];
@@ -351,7 +353,8 @@ static void setup_tiled_indices(Spkv2Context *ctx, const Uses &u) {
             for (uint16_t o = 0; o < b->output_count; o++) {
                 const Spkv2TensorRecord *w = rec(ctx, b->outputs[o]);
                 const uint64_t w0 = w->data_offset, w1 = w0 + w->size_bytes;
-                if (w->memory_class == SPKV2_MEMORY_ACTIVATION_ARENA && w0 < x1 && x0 < w1) kept = false;
+                const bool in_arena = w->role != SPKV2_ROLE_WEIGHT && w->memory_class != SPKV2_MEMORY_EXTERNAL;
+                if (in_arena && w0 < x1 && x0 < w1) kept = false;
             }
         }
         if (!kept) continue;
