@@ -39,6 +39,7 @@
 #include "conv.hpp"
 #include "igemm_split.hpp"
 #include "kernels.hpp"
+#include "parts.hpp"
 
 namespace spk::kern {
 
@@ -1480,7 +1481,8 @@ bool window_fits(const GatherSpec &gs) { return skinny_fits(gs) && gs.gather.win
 // Configuration c can run the layer.
 bool cfg_fits(int c, const GatherSpec &gs) {
     return resident_wgs(c) > 0 && (kCfgs[c].skinny_waves == 0 || skinny_fits(gs)) &&
-           (!kCfgs[c].window || window_fits(gs)) && (kCfgs[c].thin_mb == 0 || thin_fits(gs));
+           (!kCfgs[c].window || window_fits(gs)) && (kCfgs[c].thin_mb == 0 || thin_fits(gs)) &&
+           (kCfgs[c].split_threads == 0 || gs.K >= kPartsMinK);
 }
 
 std::vector<int> build_koff(const GatherSpec &gs, int BK) {

@@ -610,7 +610,7 @@ int matmul_run(Spkv2Context *ctx, const Spkv2NodeRecord *node, void *) {
     const bool small = K > 64 && tiles64 < 256;
     const int bm = small ? 32 : 64;
     const uint64_t mt_pt = (M + bm - 1) / bm, nt_pt = (N + kPtN - 1) / kPtN;
-    const bool parts_fit = M * K < limit && K * N < limit && mt_pt <= 65535;
+    const bool parts_fit = K >= kPartsMinK && M * K < limit && K * N < limit && mt_pt <= 65535;
     const bool reads_transposed = node->id < ctx->matmul_parts.size() && ctx->matmul_parts[node->id];
     const bool parts = (tiles64 >= 64 || reads_transposed) && !getenv("SPKV2_MATMUL_KSPLIT");
     if (parts_fit && (parts || trans[0] || trans[1])) {

@@ -19,6 +19,13 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsi
     l = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{s0, s1}, bf16x2));
 }
 
+// Fewest products a sum on parts takes the place of float32 multiply-adds for:
+// the three part products left out and the part sums' own roundings stay within
+// what multiply-adds round from three on (largest error relative to sum |ab|,
+// in 2^-24, multiply-adds against parts: K = 1 1.00 and 1.59, 2 1.94 and 2.65,
+// 3 2.45 and 2.12, 16 4.4 and 1.9).
+constexpr int kPartsMinK = 3;
+
 // Whether a sum of part products may differ from the float32 sum by more than
 // rounding: an infinite input or product has parts of both signs, and the
 // parts of values near the smallest float round to zero.

@@ -35,6 +35,7 @@
 #include "common.hpp"
 #include "conv.hpp"
 #include "kernels.hpp"
+#include "parts.hpp"
 
 namespace spk::kern {
 namespace {
@@ -302,7 +303,8 @@ int setup_matmul_operands(Spkv2Context *ctx, const Uses &u, bool views) {
             const Spkv2TensorRecord *o = rec(ctx, n->inputs[1 - slot]);
             const uint64_t other = o->rank >= 2 ? static_cast<uint64_t>(o->shape[o->rank - 1]) * o->shape[o->rank - 2] : ~0ull;
             if (std::max(matrix, other) >= 0x7fff0000ull / 4) continue;  // matmul_parts' offsets
-            if (!swaps || !movable_rank(ctx, u, x, rank) || u.readers[x].size() != 1 || ctx->moved[x]) continue;
+            if (!swaps || tr->shape[rank - 1 - slot] < kPartsMinK) continue;  // and its fewest products
+            if (!movable_rank(ctx, u, x, rank) || u.readers[x].size() != 1 || ctx->moved[x]) continue;
             const int xp = u.producer[x];
             if (xp < 0 || !builtin_runs(ctx, static_cast<uint32_t>(xp))) continue;
             const uint16_t op = ctx->node_records[xp].op_type;

@@ -25,7 +25,7 @@ def _close(got, a, b):
 
 
 # tiles' edges and remainders in M, N and K, on 64- and 32-row tiles
-@pytest.mark.parametrize("batch,m,n,k", [(70, 1, 1, 1), (64, 64, 64, 32), (16, 65, 127, 33), (70, 33, 66, 70),
+@pytest.mark.parametrize("batch,m,n,k", [(70, 1, 1, 3), (64, 64, 64, 32), (16, 65, 127, 33), (70, 33, 66, 70),
                                          (9, 129, 200, 31), (64, 31, 63, 130), (3, 400, 257, 101), (80, 5, 7, 64)])
 def test_matmul_parts(gpu, batch, m, n, k):
     g = models.matmul_op([batch, m, k], [batch, k, n])
@@ -34,6 +34,25 @@ def test_matmul_parts(gpu, batch, m, n, k):
         got = mdl(*xs)
         assert "matmul_parts" in mdl.kernel_name(0)
     _close(got, *xs)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("k", [1, 2, 3])
+def test_few_products(gpu, k, transposed):
+    """One or two products are summed without parts, whose left-out products
+    and extra roundings they would show: each product of K multiply-adds is
+    rounded at most K times, so |error| <= K 2^-24 sum |a b|."""
+    g = Graph("few")
+    a, b = g.input("a", [64, 96, k]), g.input("b", [64, 96, k] if transposed else [64, k, 96])
+    g.mark_output(g.matmul(a, g.transpose(g.add(b, b), [0, 2, 1]) if transposed else b))
+    xs = rng_inputs(g)
+    with Model(write_spk(g, "mi355x")) as mdl:
+        got = mdl(*xs)
+        names = [mdl.kernel_name(i) for i in range(len(g.nodes))]
+    assert any("matmul_parts" in s for s in names) == (k > 2), names
+    assert any("transpose_elided" in s for s in names) == (transposed and k > 2), names
+    x, y = (v.astype(np.float64) for v in (xs[0], 2 * np.swapaxes(xs[1], 1, 2) if transposed else xs[1]))
+    assert np.all(np.abs(got.reshape(64, 96, 96) - x @ y) <= k * 2.0 ** -24 * (np.abs(x) @ np.abs(y)))
 
 
 @pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])

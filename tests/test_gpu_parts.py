@@ -146,6 +146,20 @@ def test_parts_error_is_below_the_fp32_tiles(gpu, monkeypatch, c, k, relu):
     assert all(err[p] <= err[6] for p in PARTS_CFGS), err
 
 
+@pytest.mark.parametrize("cfg", PARTS_CFGS)
+@pytest.mark.parametrize("c", [1, 2])
+def test_few_products(gpu, monkeypatch, c, cfg):
+    """Layers of one or two products an output keep float32 multiply-adds:
+    |error| <= K 2^-24 sum |w x|."""
+    _force(monkeypatch, cfg)
+    g = models.single_conv(1, c, 64, 64, 128, 1, act=None, bias=False)
+    xs = rng_inputs(g)
+    w = g.tensors[g.nodes[0].inputs[1]].data.astype(np.float64).reshape(128, c)
+    x = xs[0].astype(np.float64).reshape(c, -1)
+    got = run_gpu(write_spk(g, "mi355x"), xs)[0].reshape(128, -1)
+    assert np.all(np.abs(got - w @ x) <= c * 2.0 ** -24 * (np.abs(w) @ np.abs(x)))
+
+
 @pytest.mark.parametrize("implicit", ["0", "1"])
 @pytest.mark.parametrize("cfg", PARTS_CFGS)
 def test_parts_special_values(gpu, monkeypatch, cfg, implicit):
