@@ -82,45 +82,10 @@ __device__ __forceinline__ unsigned tap_mask(const IgemmArgs &a, int ih, int iw)
     return v;
 }
 
-// One output's sum over k0 .. k1 - 1 in float32 multiply-adds (the packed
-// parts of a weight add up to it exactly).
-template <int BM, int BK, int MODE>
-__device__ __forceinline__ float plain_sum(const IgemmArgs &a, int m, int n, int k0, int k1) {
-    const int img = n / a.OHW, sp = n - img * a.OHW, oh = sp / a.OW, ow = sp - oh * a.OW;
-    int ihb = oh * a.sh, iwb = ow * a.sw;
-    if (MODE == kModeChk) {
-        ihb -= a.chk_ph;
-        iwb -= a.chk_pw;
-    }
-    const int col = img * a.x_img_stride + ihb * a.Wp + iwb;
-    const unsigned valid = MODE == kModeChk ? tap_mask(a, ihb, iwb) : 0u;
-    const unsigned short *w = reinterpret_cast<const unsigned short *>(a.wp);
-    float s = 0.0f;
-    for (int k = k0; k < k1; k++) {
-        if (a.koff[k] == kOobOffset) break;  // past K
-        bool in = true;  // taps outside the input are zeros
-        if (MODE == kModeChk) {
-            const unsigned t = static_cast<unsigned>(a.ktap[k]);
-            in = (valid & t) == t;
-        }
-        const int kt = k / BK, kk = k % BK, ml = m % BM;
-        const size_t at = ((((static_cast<size_t>(m / BM) * a.k_tiles + kt) * (BM / 32) + ml / 32) * (BK / 16) + kk / 16) *
-                               3 * 64 +
-                           (kk % 16 / 8) * 32 + ml % 32) *
-                              8 +
-                          kk % 8;
-        const float wv = __uint_as_float(static_cast<unsigned>(w[at]) << 16) +
-                         (__uint_as_float(static_cast<unsigned>(w[at + 512]) << 16) +
-                          __uint_as_float(static_cast<unsigned>(w[at + 1024]) << 16));
-        s = __builtin_fmaf(wv, in ? a.x[col + a.koff[k] / 4] : 0.0f, s);
-    }
-    return s;
-}
-
 }  // namespace
 
 template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, int WPE, int MODE>
-__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(IgemmArgs a) {
+__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE - (BM == 128 && MODE == kModeKvec)) conv_split_f32(IgemmArgs a) {
     constexpr int NT = 64 * WAVES_M * WAVES_N;
     constexpr int TM = BM / (32 * WAVES_M);
     constexpr int TN = BN / (32 * WAVES_N);
@@ -397,39 +362,57 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE) conv_split_f32(Ig
 
     // An infinite input or product has parts of both signs, whose sum is not
     // what a float32 sum gives, and the parts of values near the smallest
-    // float round to zero: such outputs are summed again without parts.
-    constexpr int OUTS = TM * TN * 16;
-    static_assert(OUTS <= 128, "two masks");
-    unsigned long long odd0 = 0, odd1 = 0;
+    // float round to zero: a wave's block with such an output is summed again
+    // without parts, from the same packed weights.
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             acc[i][j] += sml[i][j];
+            unsigned odd = 0;
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const float v = acc[i][j][r];
-                const int e = (i * TN + j) * 16 + r;
-                const bool odd = parts_unfit(v);
-                (e < 64 ? odd0 : odd1) |= static_cast<unsigned long long>(odd) << (e & 63);
-            }
+            for (int r = 0; r < 16; r++) odd |= static_cast<unsigned>(parts_unfit(acc[i][j][r])) << r;
+            if (!__ballot(odd != 0)) continue;
+            const int n = nt * BN + (wn * TN + j) * 32 + row;
+            const int img = n / a.OHW, sp = n - img * a.OHW, oh = sp / a.OW, ow = sp - oh * a.OW;
+            const unsigned ncol = n < a.Ntot ? (img * a.x_img_stride + oh * a.sh * a.Wp + ow * a.sw) * 4 : kOobOffset;
+            const unsigned taps = MODE == kModeChk && n < a.Ntot
+                                      ? tap_mask(a, oh * a.sh - a.chk_ph, ow * a.sw - a.chk_pw)
+                                      : 0u;
+            auto weights = [&](int k, float (&v)[8]) __attribute__((always_inline)) {
+                const int kt = min(k / BK, a.k_tiles - 1), q = k / 16 % Q;
+                const uintx4 *src = reinterpret_cast<const uintx4 *>(wbase) +
+                                    (static_cast<size_t>(kt) * (BM / 32) * Q + i * Q + q) * 3 * 64;
+                const uintx4 h = src[0], m = src[64], l = src[128];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    v[2 * e] = __uint_as_float(h[e] << 16) +
+                               (__uint_as_float(m[e] << 16) + __uint_as_float(l[e] << 16));
+                    v[2 * e + 1] = __uint_as_float(h[e] & 0xffff0000u) +
+                                   (__uint_as_float(m[e] & 0xffff0000u) + __uint_as_float(l[e] & 0xffff0000u));
+                }
+            };
+            auto inputs = [&](int k, float (&v)[8]) __attribute__((always_inline)) {
+                int ko[8], tap[8];
+                const intx4 *kp = reinterpret_cast<const intx4 *>(a.koff + k + 8 * half);
+                const intx4 *tp = reinterpret_cast<const intx4 *>(a.ktap + k + 8 * half);
+#pragma unroll
+                for (int e = 0; e < 8; e++) ko[e] = kp[e / 4][e % 4];
+                if constexpr (MODE == kModeChk) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) tap[e] = tp[e / 4][e % 4];
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    unsigned off = ncol + static_cast<unsigned>(ko[e]);  // neither wraps
+                    if constexpr (MODE == kModeChk) off = (taps & tap[e]) == static_cast<unsigned>(tap[e]) ? off : kOobOffset;
+                    v[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrs, off, 0, 0));
+                }
+            };
+            const floatx16 plain = block_sum_f32(kt0 * BK, kt1 * BK, weights, inputs);
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = odd >> r & 1 ? plain[r] : acc[i][j][r];
         }
-    if (odd0 | odd1) {
-        for (int e = 0; e < OUTS; e++) {
-            if (!((e < 64 ? odd0 : odd1) >> (e & 63) & 1)) continue;
-            const int m = mt * BM + (wm * TM + e / (TN * 16)) * 32 + 4 * half + e % 16 / 4 * 8 + e % 4;
-            const int n = nt * BN + (wn * TN + e / 16 % TN) * 32 + row;
-            if (m >= a.M || n >= a.Ntot) continue;
-            const float v = plain_sum<BM, BK, MODE>(a, m, n, kt0 * BK, kt1 * BK);
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++)
-                        if (e == (i * TN + j) * 16 + r) acc[i][j][r] = v;
-        }
-    }
     igemm_epilogue<BM, BN, 32, TM, TN, ROWMAJOR>(a, acc, mt, nt, wm, wn, lane, part, slice);
 }
 

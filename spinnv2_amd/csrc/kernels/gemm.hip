@@ -381,25 +381,36 @@ __global__ void __launch_bounds__(256) matmul_parts(MatmulArgs p) {
             for (int e = 0; e < 4; e++) acc[4 * q + e] += v[e];
         }
     }
-    // accumulator layout: column lane & 31, rows 8*(r/4) + 4*(lane/32) + r%4
-    const int n = n0 + wn * 32 + row;
+    // outputs that parts cannot give: the wave's block again without them
     unsigned odd = 0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) odd |= static_cast<unsigned>(parts_unfit(acc[r])) << r;
+    const int n = n0 + wn * 32 + row;
+    if (__ballot(odd != 0)) {
+        auto operand = [&](__amdgpu_buffer_rsrc_t rs, int ld, bool kcont, int at, int count, int k,
+                           float (&v)[8]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int kk = k + 8 * half + e;
+                const int off = (kcont ? at * ld + kk : kk * ld + at) * 4;
+                v[e] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(rs, at < count && kk < p.K ? off : 0x7fff0000, 0, 0));
+            }
+        };
+        const floatx16 plain = block_sum_f32(
+            0, p.K,
+            [&](int k, float (&v)[8]) __attribute__((always_inline)) {
+                operand(ars, lda, !TA, m0 + wm * 32 + row, p.M, k, v);
+            },
+            [&](int k, float (&v)[8]) __attribute__((always_inline)) { operand(brs, ldb, TB, n, p.N, k, v); });
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] = odd >> r & 1 ? plain[r] : acc[r];
+    }
+    // accumulator layout: column lane & 31, rows 8*(r/4) + 4*(lane/32) + r%4
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        odd |= static_cast<unsigned>(parts_unfit(acc[r])) << r;
         if (m < p.M && n < p.N) Y[static_cast<size_t>(m) * p.N + n] = acc[r];
-    }
-    if (n >= p.N) return;
-    for (; odd; odd &= odd - 1) {
-        const int r = __ffs(odd) - 1;
-        const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (m >= p.M) continue;
-        float s = 0.0f;
-        for (int k = 0; k < p.K; k++)
-            s = fmaf(A[TA ? static_cast<size_t>(k) * p.M + m : static_cast<size_t>(m) * p.K + k],
-                     B[TB ? static_cast<size_t>(n) * p.K + k : static_cast<size_t>(k) * p.N + n], s);
-        Y[static_cast<size_t>(m) * p.N + n] = s;
     }
 }
 

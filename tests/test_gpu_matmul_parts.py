@@ -118,3 +118,25 @@ def test_matmul_special_values(gpu, monkeypatch):
     fin = np.isfinite(want)
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-4)
     np.testing.assert_allclose(got[3], want[3], rtol=1e-4, atol=1e-40)
+
+
+@pytest.mark.parametrize("batch,size", [(64, 256), (1, 512)])
+def test_matmul_special_values_cost(gpu, batch, size):
+    """As for the layers: NaN in one matrix costs a few passes at most."""
+    g = models.matmul_op([batch, size, size], [batch, size, size])
+    xs = rng_inputs(g)
+    odd = xs[0].copy()
+    odd[0] = np.nan
+    took = []
+    with Model(write_spk(g, "mi355x")) as mdl:
+        mdl.set_profiling(True)
+        mdl.set_input(1, xs[1])
+        for v in (xs[0], odd):
+            mdl.set_input(0, v)
+            mdl.run()
+            assert "matmul_parts" in mdl.kernel_name(0)
+            mdl.reset_node_times()
+            for _ in range(5):
+                mdl.run()
+            took.append(mdl.node_time(0)[0])
+    assert took[1] < 10 * took[0], took

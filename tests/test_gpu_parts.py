@@ -185,6 +185,32 @@ def test_parts_special_values(gpu, monkeypatch, cfg, implicit):
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("cfg", PARTS_CFGS)
+def test_parts_special_values_cost(gpu, monkeypatch, cfg):
+    """A wave's block summed again runs about as many fp32 MFMA cycles as an
+    fp32 tile, some three times the block's own: NaN may not cost a multiple
+    of the number of outputs (a lane summing its own alone took 100 to 170
+    times a whole pass)."""
+    from spinnv2_amd.runtime import Model
+
+    _force(monkeypatch, cfg)
+    g = models.single_conv(16, 256, 14, 14, 256, 3, 1, 1, act=None)
+    x = rng_inputs(g)[0]
+    pixel, image = x.copy(), x.copy()
+    pixel[3, 5, 7, 7], image[3] = np.nan, np.nan
+    took = []
+    with Model(write_spk(g, "mi355x")) as mdl:
+        mdl.set_profiling(True)
+        for v in (x, pixel, image):
+            mdl.set_input(0, v)
+            mdl.run()
+            mdl.reset_node_times()
+            for _ in range(5):
+                mdl.run()
+            took.append(mdl.node_time(0)[0])
+    assert max(took[1:]) < 10 * took[0], took
+
+
 @pytest.mark.parametrize("scale", [1e-36, 1e-30, 1e30])
 def test_parts_scaled_inputs(gpu, monkeypatch, scale):
     """Inputs whose smaller parts would be denormal (1e-36), and far from 1."""
