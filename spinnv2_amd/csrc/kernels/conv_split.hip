@@ -14,12 +14,13 @@
 // 1.4e-7, 2.7e-7 and 8.7e-7: sixteen products are summed before a rounding
 // instead of two, and the five smaller products have an accumulator of their
 // own (in one accumulator all six would round at the sum's size: 7.3e-7 at
-// 2304).  Infinities, NaN, overflows and sums next to the smallest floats are
-// summed again in float32 multiply-adds (below).
+// 2304).  The parts are of operands scaled by 2^24, which makes them exact for
+// the smallest floats too (parts.hpp).  Infinities, NaN and overflows of scaled
+// operands or sums are summed again in float32 multiply-adds (below).
 //
 // What bounds it: per 128 x 64 x 32 step a workgroup runs 768 cycles of MFMA
 // a SIMD, loads 24 KB of weights (fragment order, straight to registers) and
-// 8 KB of activations, which it splits (5.5 VALU operations an element) into
+// 8 KB of activations, which it splits (6.5 VALU operations an element) into
 // 12 KB of LDS pieces that every wave reads.  Timed on a 14x14 3x3 layer, 256
 // channels, batch 64 (14.8 GFLOP, 392 tiles on 256 CUs): 101 us; without the
 // activations' loads 90, without splitting them 84, without the weights'
@@ -34,7 +35,8 @@ namespace {
 
 // BM x BK tiles [m_tiles][k_tiles], each [BM/32][BK/16][3 parts][64 lanes][8]
 // bf16: lane l of a 32x32x16 step holds row l & 31, k = 8 * (l >> 5) + 0..7 of
-// one part.  One thread per lane and step; ragged edges are zeros.
+// one part of 2^24 w.  One thread per lane and step; ragged edges are zeros.
+constexpr unsigned kRawWeight = 0x7f80;  // bf16 infinity, no part of a finite weight
 __global__ void __launch_bounds__(256) pack_split_kernel(const float *__restrict__ w, int M, int K, int blocks, int steps,
                                                          int k_tiles, unsigned pieces, uintx4 *__restrict__ out) {
     const unsigned id = blockIdx.x * 256u + threadIdx.x;
@@ -46,17 +48,24 @@ __global__ void __launch_bounds__(256) pack_split_kernel(const float *__restrict
     unsigned part[3][8];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        float v = m < M && k + j < K ? w[static_cast<size_t>(m) * K + k + j] : 0.0f;
+        const float raw = m < M && k + j < K ? w[static_cast<size_t>(m) * K + k + j] : 0.0f;
+        float v = raw * kPartsScale;
+        if (!(__builtin_fabsf(v) < __builtin_inff())) {
+            // 2^104 and above, infinite or NaN: an infinite part, which makes
+            // every sum it enters one that is summed again, from the weight's
+            // own bits in the other two
+            part[0][j] = kRawWeight;
+            part[1][j] = __float_as_uint(raw) >> 16;
+            part[2][j] = __float_as_uint(raw) & 0xffffu;
+            continue;
+        }
 #pragma unroll
         for (int p = 0; p < 3; p++) {
-            // to nearest; the largest floats are cut, so that none becomes
-            // infinite, and infinities and NaN have one part
-            const unsigned u = __float_as_uint(v), mag = u & 0x7fffffffu;
-            const unsigned h = mag > 0x7f800000u    ? u | 0x400000u
-                               : mag >= 0x7f7f8000u ? u
-                                                    : u + 0x7fffu + (u >> 16 & 1);
+            // to nearest; the largest floats are cut, so that none becomes infinite
+            const unsigned u = __float_as_uint(v);
+            const unsigned h = (u & 0x7fffffffu) >= 0x7f7f8000u ? u : u + 0x7fffu + (u >> 16 & 1);
             part[p][j] = h >> 16;
-            v = mag >= 0x7f800000u ? 0.0f : v - __uint_as_float(h & 0xffff0000u);
+            v -= __uint_as_float(h & 0xffff0000u);
         }
     }
 #pragma unroll
@@ -360,15 +369,13 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE - (BM == 128 && MO
         compute(0, a0, first, []() {});
     }
 
-    // An infinite input or product has parts of both signs, whose sum is not
-    // what a float32 sum gives, and the parts of values near the smallest
-    // float round to zero: a wave's block with such an output is summed again
-    // without parts, from the same packed weights.
+    // A wave's block with an output that parts cannot give (parts_unfit) is
+    // summed again without them, from the same packed weights.
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            acc[i][j] += sml[i][j];
+            acc[i][j] = (acc[i][j] + sml[i][j]) * kPartsUnscale;
             unsigned odd = 0;
 #pragma unroll
             for (int r = 0; r < 16; r++) odd |= static_cast<unsigned>(parts_unfit(acc[i][j][r])) << r;
@@ -384,12 +391,14 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE - (BM == 128 && MO
                 const uintx4 *src = reinterpret_cast<const uintx4 *>(wbase) +
                                     (static_cast<size_t>(kt) * (BM / 32) * Q + i * Q + q) * 3 * 64;
                 const uintx4 h = src[0], m = src[64], l = src[128];
+                auto whole = [](unsigned hi, unsigned mid, unsigned lo) __attribute__((always_inline)) {
+                    const float sum = __uint_as_float(hi) + (__uint_as_float(mid) + __uint_as_float(lo));
+                    return hi == kRawWeight << 16 ? __uint_as_float(mid | lo >> 16) : sum * (1.0f / kPartsScale);
+                };
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    v[2 * e] = __uint_as_float(h[e] << 16) +
-                               (__uint_as_float(m[e] << 16) + __uint_as_float(l[e] << 16));
-                    v[2 * e + 1] = __uint_as_float(h[e] & 0xffff0000u) +
-                                   (__uint_as_float(m[e] & 0xffff0000u) + __uint_as_float(l[e] & 0xffff0000u));
+                    v[2 * e] = whole(h[e] << 16, m[e] << 16, l[e] << 16);
+                    v[2 * e + 1] = whole(h[e] & 0xffff0000u, m[e] & 0xffff0000u, l[e] & 0xffff0000u);
                 }
             };
             auto inputs = [&](int k, float (&v)[8]) __attribute__((always_inline)) {

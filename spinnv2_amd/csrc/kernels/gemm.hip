@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(256) matmul_parts(MatmulArgs p) {
         step(t, 0, a1, b1, a0, b0);
         if (t + 1 < tiles) step(t + 1, 1, a0, b0, a1, b1);
     }
-    acc += sml;
+    acc = (acc + sml) * kPartsUnscale;
     if constexpr (BM == 32) {
         // the second k half's sums, 16 floats a lane, through LDS
         floatx4 *red = reinterpret_cast<floatx4 *>(&As[0][0][0][0]);

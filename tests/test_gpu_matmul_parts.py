@@ -140,3 +140,18 @@ def test_matmul_special_values_cost(gpu, batch, size):
                 mdl.run()
             took.append(mdl.node_time(0)[0])
     assert took[1] < 10 * took[0], took
+
+
+@pytest.mark.parametrize("batch", [1, 64])  # 32- and 64-row tiles
+@pytest.mark.parametrize("a_scale,b_scale", [(1e-37, 1.0), (1.0, 2e-38), (1e-41, 1e20), (1e12, 1e-36), (1e-43, 1e30),
+                                             (1e33, 1e-30), (1e12, 1e16)])
+def test_matmul_scaled_operands(gpu, batch, a_scale, b_scale):
+    """As for the layers: operands near either end of the float range."""
+    m, n, k = (512, 512, 70) if batch == 1 else (40, 50, 70)
+    g = models.matmul_op([batch, m, k], [batch, k, n])
+    a, b = ((x.astype(np.float64) * s).astype(np.float32) for x, s in zip(rng_inputs(g), (a_scale, b_scale)))
+    with Model(write_spk(g, "mi355x")) as mdl:
+        got = mdl(a, b).reshape(batch, m, n).astype(np.float64)
+        assert "matmul_parts" in mdl.kernel_name(0)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(got - a @ b) <= (k / 8 + 16) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + 2.0 ** -150)

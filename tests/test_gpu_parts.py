@@ -222,3 +222,25 @@ def test_parts_scaled_inputs(gpu, monkeypatch, scale):
     cols = _columns(xs[0], 3, 1, [1, 1, 1, 1])
     want, size = (w @ cols).ravel(), (np.abs(w) @ np.abs(cols)).ravel()
     assert np.all(np.abs(got - want) <= 288 * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("cfg", PARTS_CFGS)
+@pytest.mark.parametrize("w_scale,x_scale", [(1e-37, 1.0), (2e-38, 1.0), (1e-41, 1e20), (1e12, 1e-36), (1e20, 1e-38),
+                                             (1e30, 1e-43), (1e-30, 1e33), (1e33, 1e-30), (1e16, 1e12)])
+def test_parts_scaled_operands(gpu, monkeypatch, w_scale, x_scale, cfg):
+    """Operands whose smaller parts would lie below the smallest bf16, and
+    those that do not stay finite when scaled for the split (1e33, and sums of
+    1e28): the bound of the other tests, and half of the smallest float."""
+    _force(monkeypatch, cfg)
+    rng = np.random.default_rng(9)
+    w = (rng.standard_normal((40, 32, 3, 3)) * w_scale).astype(np.float32)
+    x = (rng.standard_normal((1, 32, 6, 7)) * x_scale).astype(np.float32)
+    g = Graph("scaled")
+    g.mark_output(g.conv(g.input("x", list(x.shape)), w, np.zeros(40, np.float32), pad=1))
+    cols, w2 = _columns(x, 3, 1, [1, 1, 1, 1])[0], w.astype(np.float64).reshape(40, -1)
+    want, size = w2 @ cols, np.abs(w2) @ np.abs(cols)
+    for implicit in ("0", "1"):
+        monkeypatch.setenv("SPKV2_IMPLICIT_PAD", implicit)
+        got = run_gpu(write_spk(g, "mi355x"), [x])[0].astype(np.float64).reshape(want.shape)
+        err = np.abs(got - want)
+        assert np.all(err <= (288 / 8 + 16) * 2.0 ** -24 * size + 2.0 ** -150), float(np.max(err / size) * 2 ** 24)
