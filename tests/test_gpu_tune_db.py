@@ -163,3 +163,38 @@ def test_deterministic_tuner_is_bit_reproducible_outside_the_table(gpu):
         runs.append(json.loads(out.stdout.strip().splitlines()[-1]))
     print("tile picks that differ:", [(a, b) for a, b in zip(runs[0]["names"], runs[1]["names"]) if a != b])
     assert runs[0]["sha"] == runs[1]["sha"]
+
+
+def test_tuner_times_ordinary_operands(gpu, monkeypatch, capfd):
+    """The tuner's time of its choice is that of ordinary values (at which
+    the chip lowers its clock: 20% here), not that of zeros, which is below
+    the layer's node time on zeros by what the node's events take."""
+    import numpy as np
+
+    from spinnv2_amd.runtime import Model
+    from spinnv2_amd.spk import models, write_spk
+
+    for k in ("SPKV2_TUNE_DB", "SPKV2_CONV_CFG", "SPKV2_CONV_SPLITK", "SPKV2_CONV_HYBRID", "SPKV2_CONV_TUNE"):
+        monkeypatch.delenv(k, raising=False)
+    monkeypatch.setenv("SPKV2_TUNE_LOG", "1")
+    monkeypatch.setenv("SPKV2_TUNE_TIE", "0")  # the fastest candidate, first in the log
+    took = {}
+    for name in ("ordinary", "zeros"):
+        g = models.single_conv(48, 272, 29, 29, 256, 3, act=None)
+        x = np.random.default_rng(1).standard_normal((48, 272, 29, 29)).astype(np.float32)
+        if name == "zeros":
+            x[:] = 0
+            g.tensors[g.nodes[0].inputs[1]].data[:] = 0
+        with Model(write_spk(g, "mi355x")) as mdl:
+            mdl.set_profiling(True)
+            mdl.set_input(0, x)
+            for _ in range(10):
+                mdl.run()
+            mdl.reset_node_times()
+            for _ in range(30):
+                mdl.run()
+            ms, runs = mdl.node_time(0)[:2]
+            took[name] = 1e3 * ms / runs
+    tuned = [line for line in capfd.readouterr().err.splitlines() if line.startswith("[tune]   ")]
+    best = float(tuned[0].split()[-1])
+    assert best > took["zeros"], (best, took)
