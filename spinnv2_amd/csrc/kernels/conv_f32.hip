@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(256) conv_igemm_f32(IgemmArgs a) {
     }
 #define IGEMM_LOAD_B(KT, BR)                                                                                         \
     {                                                                                                                \
-        /* the table has two tiles of out-of-range entries past Kpad */                                           \
+        /* the table goes kTilesPastK tiles past Kpad */                                                          \
         const int *ko = a.koff + (KT) * BK + bgrp * KPT;                                                              \
         if constexpr (KVEC) {                                                                                        \
             /* the four k of a quad are all below K or all past it (K % 4 == 0) */                                  \
@@ -1487,9 +1487,7 @@ bool cfg_fits(int c, const GatherSpec &gs) {
 
 std::vector<int> build_koff(const GatherSpec &gs, int BK) {
     const int kpad = (gs.K + BK - 1) / BK * BK;
-    // three extra tiles of out-of-range entries: the pipelines read up to
-    // three tiles past the last one
-    std::vector<int> koff(static_cast<size_t>(kpad + 3 * BK), kOobOffset);
+    std::vector<int> koff(static_cast<size_t>(kpad + kTilesPastK * BK), kOobOffset);
     for (int k = 0; k < gs.K; k++) koff[k] = gs.koff(k);
     return koff;
 }
@@ -2340,7 +2338,7 @@ static int use_implicit_padding(ConvPlan *plan) {
         const double copied = 4e-6 * g.N * g.C * (static_cast<double>(g.H) * g.W + static_cast<double>(plan->Hp) * plan->Wp);
         if ((plan->BM < 64 ? 0.2 : 0.1) * gathered > 3.0 + 0.17 * copied) return 0;
     }
-    const size_t entries = static_cast<size_t>(plan->Kpad) + 3 * BK;  // as build_koff: three tiles past Kpad
+    const size_t entries = static_cast<size_t>(plan->Kpad) + kTilesPastK * BK;  // as build_koff
     std::vector<int> koff(entries, kOobOffset), ktap(entries, parts ? -1 : 0x7fff7fff);
     for (int k = 0; k < K; k++) {
         const int c = k / (g.KH * g.KW), r = k % (g.KH * g.KW);

@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N, WPE - (BM == 128 && MO
                 for (int p = 0; p < 3; p++) ax[i][q][p] = src[((i * Q + q) * 3 + p) * 64];
     };
     // The k offsets are read one tile ahead of the loads that use them (the
-    // table has three tiles of out-of-range entries past K), in two sets taken
+    // table goes kTilesPastK tiles past K), in two sets taken
     // in turn: a scalar load in flight makes every wait for LDS wait for it
     // too, so it is issued ahead of the step's vector loads, which cover it
     // (72 to 100 channels, stride 2, at 75x57, batch 5 33.2 -> 30.8 us; it also

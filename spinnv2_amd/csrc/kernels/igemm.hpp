@@ -13,10 +13,15 @@ constexpr int kBufferWord3 = 0x00020000;
 // still does not wrap when a valid offset is added to it
 constexpr int kOobOffset = 0x7fff0000;
 
+// Tiles of out-of-range entries that a k -> offset table (and a tap table) has
+// past the last one: conv_split_f32 reads offsets three tiles ahead, the others
+// two.
+constexpr int kTilesPastK = 3;
+
 struct IgemmArgs {
     const float *__restrict__ x;     // B-operand source: NCHW input, zero-padded when the conv pads
     const float *__restrict__ wp;    // [m_tiles][k_tiles] BM x BK tiles in MFMA fragment order
-    const int *__restrict__ koff;    // [Kpad + 2*BK] byte offset of k = (c, kh, kw) in x, kOobOffset past K
+    const int *__restrict__ koff;    // [Kpad + kTilesPastK * BK] byte offset of k = (c, kh, kw) in x, kOobOffset past K
     const float *__restrict__ bias;  // [M] or null
     const float *__restrict__ res;   // like y, or null
     float *__restrict__ y;
@@ -45,8 +50,8 @@ struct IgemmArgs {
     // (kh, kw) = (tap / sk_KW, tap % sk_KW) kh * sk_tap_h + kw * sk_tap_w
     // elements past tap 0
     int sk_C, sk_cstride, sk_KW, sk_tap_h, sk_tap_w;
-    // implicit padding (kModeChk): per-k tap table ((kh*dh) << 16 | kw*dw,
-    // 0x7fff7fff past K), the unpadded input's extent and the padding
+    // implicit padding (kModeChk): per-k tap table of koff's size ((kh*dh) <<
+    // 16 | kw*dw, 0x7fff7fff past K), the unpadded input's extent and the padding
     const int *__restrict__ ktap;
     int chk_H, chk_W, chk_ph, chk_pw;
     int chk_KH, chk_KW, chk_dh, chk_dw;  // conv_split_f32: its ktap entry is bits kh and 16 + kw, all ones past K
