@@ -15,7 +15,7 @@ import pytest
 from spinnv2_amd.spk import models, write_spk
 from spinnv2_amd.spk.graph import Graph
 
-from .helpers import rng_inputs, run_gpu
+from .helpers import FP32_TOL, rng_inputs, run_gpu, run_oracle, tnorm_err
 
 pytestmark = pytest.mark.gpu
 
@@ -244,3 +244,35 @@ def test_parts_scaled_operands(gpu, monkeypatch, w_scale, x_scale, cfg):
         got = run_gpu(write_spk(g, "mi355x"), [x])[0].astype(np.float64).reshape(want.shape)
         err = np.abs(got - want)
         assert np.all(err <= (288 / 8 + 16) * 2.0 ** -24 * size + 2.0 ** -150), float(np.max(err / size) * 2 ** 24)
+
+
+# (C, H, W, Cout, k, stride, pads, dilation, residual, activation): dilation,
+# asymmetric padding, the most taps a side that the tap table holds and one more
+IPAD_CASES = [
+    (16, 13, 11, 40, 3, 1, [1, 1, 1, 1], 1, True, "Relu"),
+    (8, 20, 20, 24, 3, 1, [2, 2, 2, 2], 2, True, None),
+    (8, 21, 18, 70, 3, 2, [3, 0, 1, 5], 3, False, "Silu"),
+    (3, 20, 17, 33, 5, 1, [8, 4, 0, 6], 2, False, "Relu"),
+    (2, 19, 16, 33, 15, 1, [7, 7, 7, 7], 1, False, "Silu"),
+    (2, 19, 18, 33, 16, 1, [8, 8, 7, 7], 1, False, "Relu"),
+]
+
+
+@pytest.mark.parametrize("implicit", ["1", "0"])
+@pytest.mark.parametrize("cfg", PARTS_CFGS)
+@pytest.mark.parametrize("case", IPAD_CASES, ids=[f"ipad{i}" for i in range(len(IPAD_CASES))])
+def test_parts_implicit_padding(gpu, monkeypatch, case, cfg, implicit):
+    from spinnv2_amd.runtime import Model
+
+    _force(monkeypatch, cfg)
+    monkeypatch.setenv("SPKV2_IMPLICIT_PAD", implicit)
+    c, h, w, m, k, s, pads, d, res, act = case
+    g = models.single_conv(2, c, h, w, m, k, s, dilation=d, act=act, residual=res, pads=pads)
+    blob = write_spk(g, "mi355x")
+    xs = rng_inputs(g)
+    with Model(blob) as mdl:
+        got = mdl(*xs)
+        name = mdl.kernel_name(0)
+    assert "conv_split_f32" in name, name
+    assert (",ipad" in name) == (implicit == "1" and k <= 15), name
+    assert tnorm_err(got, run_oracle(blob, xs)[0]) <= FP32_TOL
