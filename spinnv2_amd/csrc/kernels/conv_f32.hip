@@ -1464,6 +1464,10 @@ struct GatherSpec {
     std::function<int(int)> koff;  // byte offset of k < K
     std::string key;   // everything the timing depends on
     GatherGeom gather;  // the same rule per tap (skinny kernel), 16-byte k loads (KVEC)
+    // the layer pads its own input (Hp x Wp planes, pt / pl at the top / left)
+    // or checks its taps
+    bool copied = false;
+    int Hp = 0, pt = 0, pl = 0;
 };
 
 // The skinny kernel takes a layer whose channels per tap are a multiple of
@@ -1492,7 +1496,97 @@ std::vector<int> build_koff(const GatherSpec &gs, int BK) {
     return koff;
 }
 
+// Implicit padding.  A padded conv whose input no producer hands over in
+// padded form, and whose gather per output pixel is short (C*KH*KW <= 160:
+// RGB stems, 3x3 convs of up to 16 channels), reads the unpadded input with
+// every tap bounds-checked (kModeChk) instead of copying it into a
+// zero-padded buffer first: the k -> offset table is rebuilt for the
+// unpadded input, a tap table gives (kh*dh, kw*dw) per k, and the padded
+// copy's workspace is dropped.  For longer gathers the checks on every
+// element cost more than the copy saves (a 64-channel 3x3 conv at 80x80,
+// batch 16: 170 against 124 us with its copy), so they keep the copy; so
+// do the skinny kernel (it reads a padded input) and inputs 16384 or more
+// rows or columns tall (the tap table packs a tap into 16 bits).  The tiles
+// on bf16 parts check a tap with one and and one compare (tap_mask): per
+// million elements gathered that is about 0.1 us, twice that with 32 rows, and
+// a copy costs about 3 us and 0.17 us per MB read and written, so they take
+// the checks where those come out cheaper.  With the copy and without, in us:
+// 14x14, 256 channels, 128 rows, batch 64 110 and 104; 64 channels at 80x80,
+// 64 rows, batch 16 74 and 67; 72 to 100 channels at 75x57, stride 2 29.6 and
+// 23.6; on the other side 256 channels at 56x56, 128 rows, batch 16 330 and
+// 341; 14x14, 64 rows, batch 64 133 and 141; 7x7 taps over 240 channels at
+// 30x201, 32 rows 106 and 118.
+// SPKV2_IMPLICIT_PAD=0 keeps the copy everywhere, =1 takes the checks
+// wherever they apply.
+bool takes_checks(const ConvGeom &g, int cfg, int Hp, int Wp) {
+    const TileCfg &t = kCfgs[cfg];
+    if (t.skinny_waves > 0 || t.thin_mb > 0) return false;
+    if (g.H >= 16384 || g.W >= 16384 || (g.KH - 1) * g.dh >= 32768 || (g.KW - 1) * g.dw >= 32768) return false;
+    const char *e = getenv("SPKV2_IMPLICIT_PAD");
+    if (e && e[0] == '0') return false;
+    const bool parts = t.split_threads > 0;
+    if (parts && (g.KH > 15 || g.KW > 15)) return false;  // its tap table has 15 bits a side
+    const int K = g.C * g.KH * g.KW;
+    if (!(e && e[0] == '1') && K > 160) {
+        if (!parts) return false;
+        const double gathered = 1e-6 * K * g.N * g.OH * g.OW * ((g.M + t.BM - 1) / t.BM);
+        const double copied = 4e-6 * g.N * g.C * (static_cast<double>(g.H) * g.W + static_cast<double>(Hp) * Wp);
+        if ((t.BM < 64 ? 0.2 : 0.1) * gathered > 3.0 + 0.17 * copied) return false;
+    }
+    return true;
+}
+
+// Its tables, for configuration cfg.
+struct CheckedTables {
+    std::vector<int> koff, ktap;
+};
+CheckedTables checked_tables(const ConvGeom &g, int cfg) {
+    const bool parts = kCfgs[cfg].split_threads > 0;
+    const int BK = kCfgs[cfg].BK, K = g.C * g.KH * g.KW;
+    const size_t entries = static_cast<size_t>((K + BK - 1) / BK + kTilesPastK) * BK;  // as build_koff
+    CheckedTables t{std::vector<int>(entries, kOobOffset), std::vector<int>(entries, parts ? -1 : 0x7fff7fff)};
+    for (int k = 0; k < K; k++) {
+        const int c = k / (g.KH * g.KW), r = k % (g.KH * g.KW);
+        const int th = (r / g.KW) * g.dh, tw = (r % g.KW) * g.dw;
+        t.koff[k] = ((c * g.H + th) * g.W + tw) * 4;
+        t.ktap[k] = parts ? (1 << (r / g.KW)) | (1 << (16 + r % g.KW)) : (th << 16) | tw;
+    }
+    return t;
+}
+
+GatherGeom checked_gather(const ConvGeom &g, GatherGeom gather, const void *ktap) {
+    gather.ktap = static_cast<const int *>(ktap);
+    gather.chk = true;
+    gather.chk_H = g.H;
+    gather.chk_W = g.W;
+    gather.chk_ph = g.ph;
+    gather.chk_pw = g.pw;
+    return gather;
+}
+
 }  // namespace
+
+// x (images x_img elements apart) into the zero-padded planes xp.
+static int launch_pad(hipStream_t st, const ConvGeom &g, const float *x, float *xp, int Hp, int Wp, int pt, int pl,
+                      size_t x_img) {
+    PadArgs pa{};
+    pa.x = x;
+    pa.xp = xp;
+    pa.total = static_cast<unsigned>(g.N * g.C) * static_cast<unsigned>(Hp * Wp);  // below 2^29 (plan_igemm_f32)
+    pa.C = g.C;
+    pa.H = g.H;
+    pa.W = g.W;
+    pa.Hp = Hp;
+    pa.Wp = Wp;
+    pa.pt = pt;
+    pa.pl = pl;
+    pa.x_img = x_img;
+    div_magic(static_cast<unsigned>(Hp * Wp), &pa.plane_m, &pa.plane_s);
+    div_magic(static_cast<unsigned>(Wp), &pa.wp_m, &pa.wp_s);
+    div_magic(static_cast<unsigned>(g.C), &pa.c_m, &pa.c_s);
+    hipLaunchKernelGGL(pad_nchw, dim3((pa.total / 4 + 256) / 256), dim3(256), 0, st, pa);
+    return launch_status("pad_nchw");
+}
 
 // Launches the implicit GEMM of configuration cfg with tile counts tc over
 // an already prepared (padded) B source, then the split-K epilogue.
@@ -1755,7 +1849,8 @@ __global__ void __launch_bounds__(256) fill_operands(unsigned *__restrict__ p, s
 }
 
 // Times every candidate (configuration x split-K) the model does not rule
-// out on scratch buffers of the layer's real shape, and returns the fastest
+// out on scratch buffers of the layer's real shape, with the copy or the checks
+// of a layer that pads its own input, and returns the fastest
 // (cfg, split request).  Results are cached per shape for the process, so
 // every context sees the same choice for the same layer.  Returns false
 // when the device could not be used (the caller then trusts the model).
@@ -1840,6 +1935,22 @@ bool tune_tiles(hipStream_t st, const ConvGeom &g, const GatherSpec &gs, int *cf
     float *ws = static_cast<float *>(tb.alloc(ws_bytes));
     float *bias = g.has_bias ? static_cast<float *>(tb.alloc(static_cast<size_t>(g.M) * 4)) : nullptr;
     float *res = g.has_res ? static_cast<float *>(tb.alloc(y_bytes)) : nullptr;
+    // a layer that pads its own input: its unpadded input, and each candidate
+    // with the padding it will run with
+    float *xu = gs.copied ? static_cast<float *>(tb.alloc(static_cast<size_t>(g.x_elems) * 4)) : nullptr;
+    auto checks = [&](const Cand &cd) { return gs.copied && takes_checks(g, cd.cfg, gs.Hp, gs.Wp); };
+    std::map<std::pair<int, bool>, std::pair<int *, int *>> checked;  // (BK, on parts) -> koff, ktap
+    for (const Cand &cd : keep) {
+        const std::pair<int, bool> kind{kCfgs[cd.cfg].BK, kCfgs[cd.cfg].split_threads > 0};
+        if (!checks(cd) || checked.count(kind)) continue;
+        const CheckedTables t = checked_tables(g, cd.cfg);
+        const size_t bytes = t.koff.size() * sizeof(int);
+        int *const ko = static_cast<int *>(tb.alloc(bytes)), *const kt = static_cast<int *>(tb.alloc(bytes));
+        if (!ko || !kt || hipMemcpy(ko, t.koff.data(), bytes, hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy(kt, t.ktap.data(), bytes, hipMemcpyHostToDevice) != hipSuccess)
+            return untimed();
+        checked[kind] = {ko, kt};
+    }
     int *koff[4] = {nullptr, nullptr, nullptr, nullptr};  // BK 16, 32, 64, 128
     for (int i = 0; i < 4; i++) {
         const std::vector<int> kv = build_koff(gs, 16 << i);
@@ -1847,7 +1958,8 @@ bool tune_tiles(hipStream_t st, const ConvGeom &g, const GatherSpec &gs, int *cf
         if (koff[i] && hipMemcpy(koff[i], kv.data(), kv.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
             koff[i] = nullptr;
     }
-    if (!xs || !wp || !y || !ws || (g.has_bias && !bias) || (g.has_res && !res) || !koff[0] || !koff[1] || !koff[2] || !koff[3])
+    if (!xs || !wp || !y || !ws || (g.has_bias && !bias) || (g.has_res && !res) || (gs.copied && !xu) || !koff[0] ||
+        !koff[1] || !koff[2] || !koff[3])
         return untimed();
     auto fill = [&](float *p, size_t bytes) {
         if (p)
@@ -1855,7 +1967,7 @@ bool tune_tiles(hipStream_t st, const ConvGeom &g, const GatherSpec &gs, int *cf
                                reinterpret_cast<unsigned *>(p), bytes / 4);
         return launch_status("fill_operands") == 0;
     };
-    if (!fill(xs, gs.x_bytes) || !fill(wp, wpack_bytes) || !fill(bias, static_cast<size_t>(g.M) * 4) ||
+    if (!fill(xs, gs.x_bytes) || !fill(xu, static_cast<size_t>(g.x_elems) * 4) || !fill(wp, wpack_bytes) || !fill(bias, static_cast<size_t>(g.M) * 4) ||
         !fill(res, y_bytes))
         return untimed();
 
@@ -1868,10 +1980,22 @@ bool tune_tiles(hipStream_t st, const ConvGeom &g, const GatherSpec &gs, int *cf
         const int bk = kCfgs[cd.cfg].BK;
         const int *ko = koff[bk == 16 ? 0 : bk == 32 ? 1 : bk == 64 ? 2 : 3];
         if (hipEventRecord(e0, st) != hipSuccess) return 1e300;
-        for (int r = 0; r < reps; r++)
-            if (launch_igemm(st, cd.cfg, cd.tc, g, gs.Wp, xs, gs.x_bytes, gs.x_img_stride, wp, ko, bias, res, y, 1.0f,
-                             ws, gs.gather) != 0)
-                return 1e300;
+        const int x_img = g.C * g.H * g.W;
+        for (int r = 0; r < reps; r++) {
+            int rc = 0;
+            if (checks(cd)) {
+                const auto &[cko, ckt] = checked[{bk, kCfgs[cd.cfg].split_threads > 0}];
+                rc = launch_igemm(st, cd.cfg, cd.tc, g, g.W, xu, static_cast<int>(g.x_elems * 4), x_img, wp, cko, bias,
+                                  res, y, 1.0f, ws, checked_gather(g, gs.gather, ckt));
+            } else {
+                if (gs.copied)
+                    rc = launch_pad(st, g, xu, xs, gs.Hp, gs.Wp, gs.pt, gs.pl, static_cast<size_t>(x_img));
+                if (rc == 0)
+                    rc = launch_igemm(st, cd.cfg, cd.tc, g, gs.Wp, xs, gs.x_bytes, gs.x_img_stride, wp, ko, bias, res,
+                                      y, 1.0f, ws, gs.gather);
+            }
+            if (rc != 0) return 1e300;
+        }
         if (hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) return 1e300;
         float ms = 0.0f;
         if (hipEventElapsedTime(&ms, e0, e1) != hipSuccess) return 1e300;
@@ -1919,12 +2043,12 @@ bool tune_tiles(hipStream_t st, const ConvGeom &g, const GatherSpec &gs, int *cf
     tuned_store(gs.key, keep[pick].cfg, keep[pick].split);
     if (const char *e = getenv("SPKV2_TUNE_LOG"))
         if (e[0] == '1') {
-            // every timed candidate, fastest first: config, split request,
-            // model estimate and measured time (us)
+            // every timed candidate, fastest first: config, the padding of its
+            // input, split request, model estimate and measured time (us)
             fprintf(stderr, "[tune] %s -> cfg %d split %d\n", gs.key.c_str(), keep[pick].cfg, keep[pick].split);
             for (const Cand &cd : keep)
-                fprintf(stderr, "[tune]   %-10s split %4d splitk %2d  model %7.2f  time %7.2f\n", kCfgs[cd.cfg].name,
-                        cd.split, cd.tc.splitk, cd.model, cd.t);
+                fprintf(stderr, "[tune]   %-10s%s split %4d splitk %2d  model %7.2f  time %7.2f\n", kCfgs[cd.cfg].name,
+                        checks(cd) ? ",ipad" : gs.copied ? ",copy" : "", cd.split, cd.tc.splitk, cd.model, cd.t);
         }
     return true;
 }
@@ -2136,13 +2260,30 @@ static bool padded_extent(const ConvGeom &g, int *Hp, int *Wp) {
     return g.ph > 0 || g.pw > 0 || hspan - g.ph > g.H || wspan - g.pw > g.W;
 }
 
+// Where a padded conv's input can come from in padded form: the plan of the conv
+// that makes it, directly or through a channel Split that cuts channels m0 on,
+// and the tensor's readers.  No producer: the conv pads its own input.
+struct PadSource {
+    ConvPlan *producer = nullptr;
+    int m0 = 0, readers = 0;
+    bool via_split = false;
+};
+
+// The producer hands this tensor to an earlier reader already, in the padded
+// geometry and channel range that `plan` needs, too.
+static bool shares_pad(const PadSource &src, const ConvPlan *plan) {
+    const ConvPlan *pp = src.producer;
+    return pp->pad_out && pp->pad_Hp == plan->Hp && pp->pad_Wp == plan->Wp && pp->pad_pt == plan->pt &&
+           pp->pad_pl == plan->pl && pp->pad_m0 == src.m0 && pp->pad_C == (src.via_split ? plan->g.C : 0);
+}
+
 // Plans an fp32 implicit GEMM for convolution g (group 1) with weights
 // w_host[M][C*KH*KW].  When some tap falls outside the input, the input is
 // first copied into a zero-padded buffer so the kernel needs no bounds tests;
 // min_Hp / min_Wp enlarge that buffer's planes (a geometry shared with the
 // other padded readers of the same input).
 int plan_igemm_f32(hipStream_t st, const ConvGeom &g, const float *w_host, ConvPlan *plan, int min_Hp = 0,
-                   int min_Wp = 0) {
+                   int min_Wp = 0, const PadSource &src = {}) {
     const int K = g.C * g.KH * g.KW;
     int ext_h = 0, ext_w = 0;
     plan->padded = padded_extent(g, &ext_h, &ext_w);
@@ -2165,6 +2306,10 @@ int plan_igemm_f32(hipStream_t st, const ConvGeom &g, const float *w_host, ConvP
         return ((c * Hp + kh * g.dh) * Wp + kw * g.dw) * 4;
     };
     gs.key = shape_key("conv", g, plan, gs.x_img_stride);
+    gs.copied = plan->padded && !(src.producer && (!src.producer->pad_out || shares_pad(src, plan)));
+    gs.Hp = plan->Hp;
+    gs.pt = plan->pt;
+    gs.pl = plan->pl;
     gs.gather.C = g.C;
     gs.gather.cstride = Hp * Wp;
     gs.gather.KW = g.KW;
@@ -2271,26 +2416,10 @@ static int run_igemm_impl(Spkv2Context *ctx, const ConvPlan *p, const float *x, 
         x_img_stride = g.C * p->Hp * p->Wp;
     } else if (p->padded) {
         float *xp = reinterpret_cast<float *>(wsb);
-        const unsigned planes = static_cast<unsigned>(g.N * g.C);
-        PadArgs pa{};
-        pa.x = x;
-        pa.xp = xp;
-        pa.total = planes * static_cast<unsigned>(p->Hp * p->Wp);  // below 2^29 (plan_igemm_f32)
-        pa.C = g.C;
-        pa.H = g.H;
-        pa.W = g.W;
-        pa.Hp = p->Hp;
-        pa.Wp = p->Wp;
-        pa.pt = p->pt;
-        pa.pl = p->pl;
-        pa.x_img = static_cast<size_t>(x_img_stride);
-        div_magic(static_cast<unsigned>(p->Hp * p->Wp), &pa.plane_m, &pa.plane_s);
-        div_magic(static_cast<unsigned>(p->Wp), &pa.wp_m, &pa.wp_s);
-        div_magic(static_cast<unsigned>(g.C), &pa.c_m, &pa.c_s);
-        hipLaunchKernelGGL(pad_nchw, dim3((pa.total / 4 + 256) / 256), dim3(256), 0, ctx->stream, pa);
-        if (int rc = launch_status("pad_nchw")) return rc;
+        if (int rc = launch_pad(ctx->stream, g, x, xp, p->Hp, p->Wp, p->pt, p->pl, static_cast<size_t>(x_img_stride)))
+            return rc;
         xs = xp;
-        x_bytes = static_cast<int>(static_cast<size_t>(planes) * p->Hp * p->Wp * 4);
+        x_bytes = static_cast<int>(static_cast<size_t>(g.N) * g.C * p->Hp * p->Wp * 4);
         x_img_stride = g.C * p->Hp * p->Wp;
     }
     float *ws = p->workspace > 0 ? reinterpret_cast<float *>(wsb + p->pad_bytes) : nullptr;
@@ -2300,66 +2429,19 @@ static int run_igemm_impl(Spkv2Context *ctx, const ConvPlan *p, const float *x, 
                         give && !p->y_needed ? nullptr : y, alpha, ws, p->gather, give ? p : nullptr, yl);
 }
 
-// Implicit padding.  A padded conv whose input no producer hands over in
-// padded form, and whose gather per output pixel is short (C*KH*KW <= 160:
-// RGB stems, 3x3 convs of up to 16 channels), reads the unpadded input with
-// every tap bounds-checked (kModeChk) instead of copying it into a
-// zero-padded buffer first: the k -> offset table is rebuilt for the
-// unpadded input, a tap table gives (kh*dh, kw*dw) per k, and the padded
-// copy's workspace is dropped.  For longer gathers the checks on every
-// element cost more than the copy saves (a 64-channel 3x3 conv at 80x80,
-// batch 16: 170 against 124 us with its copy), so they keep the copy; so
-// do the skinny kernel (it reads a padded input) and inputs 16384 or more
-// rows or columns tall (the tap table packs a tap into 16 bits).  The tiles
-// on bf16 parts check a tap with one and and one compare (tap_mask): per
-// million elements gathered that is about 0.1 us, twice that with 32 rows, and
-// a copy costs about 3 us and 0.17 us per MB read and written, so they take
-// the checks where those come out cheaper.  With the copy and without, in us:
-// 14x14, 256 channels, 128 rows, batch 64 110 and 104; 64 channels at 80x80,
-// 64 rows, batch 16 74 and 67; 72 to 100 channels at 75x57, stride 2 29.6 and
-// 23.6; on the other side 256 channels at 56x56, 128 rows, batch 16 330 and
-// 341; 14x14, 64 rows, batch 64 133 and 141; 7x7 taps over 240 channels at
-// 30x201, 32 rows 106 and 118.
-// SPKV2_IMPLICIT_PAD=0 keeps the copy everywhere, =1 takes the checks
-// wherever they apply.
 static int use_implicit_padding(ConvPlan *plan) {
     const ConvGeom &g = plan->g;
-    if (!plan->padded || plan->pad_in || kCfgs[plan->cfg].skinny_waves > 0 || kCfgs[plan->cfg].thin_mb > 0) return 0;
-    if (g.H >= 16384 || g.W >= 16384 || (g.KH - 1) * g.dh >= 32768 || (g.KW - 1) * g.dw >= 32768) return 0;
-    const char *e = getenv("SPKV2_IMPLICIT_PAD");
-    if (e && e[0] == '0') return 0;
-    const bool parts = kCfgs[plan->cfg].split_threads > 0;
-    if (parts && (g.KH > 15 || g.KW > 15)) return 0;  // its tap table has 15 bits a side
-    const int BK = plan->BK;
-    const int K = g.C * g.KH * g.KW;
-    if (!(e && e[0] == '1') && K > 160) {
-        if (!parts) return 0;
-        const double gathered = 1e-6 * K * g.N * g.OH * g.OW * ((g.M + plan->BM - 1) / plan->BM);
-        const double copied = 4e-6 * g.N * g.C * (static_cast<double>(g.H) * g.W + static_cast<double>(plan->Hp) * plan->Wp);
-        if ((plan->BM < 64 ? 0.2 : 0.1) * gathered > 3.0 + 0.17 * copied) return 0;
-    }
-    const size_t entries = static_cast<size_t>(plan->Kpad) + kTilesPastK * BK;  // as build_koff
-    std::vector<int> koff(entries, kOobOffset), ktap(entries, parts ? -1 : 0x7fff7fff);
-    for (int k = 0; k < K; k++) {
-        const int c = k / (g.KH * g.KW), r = k % (g.KH * g.KW);
-        const int th = (r / g.KW) * g.dh, tw = (r % g.KW) * g.dw;
-        koff[k] = ((c * g.H + th) * g.W + tw) * 4;
-        ktap[k] = parts ? (1 << (r / g.KW)) | (1 << (16 + r % g.KW)) : (th << 16) | tw;
-    }
+    if (!plan->padded || plan->pad_in || !takes_checks(g, plan->cfg, plan->Hp, plan->Wp)) return 0;
+    const CheckedTables t = checked_tables(g, plan->cfg);
     void *kt = nullptr, *tt = nullptr;
-    if (int rc = upload_koff(koff, &kt)) return rc;
-    if (int rc = upload_koff(ktap, &tt)) {
+    if (int rc = upload_koff(t.koff, &kt)) return rc;
+    if (int rc = upload_koff(t.ktap, &tt)) {
         (void)hipFree(kt);
         return rc;
     }
     if (plan->ktab) (void)hipFree(plan->ktab);
     plan->ktab = kt;
-    plan->gather.ktap = static_cast<const int *>(tt);
-    plan->gather.chk = true;
-    plan->gather.chk_H = g.H;
-    plan->gather.chk_W = g.W;
-    plan->gather.chk_ph = g.ph;
-    plan->gather.chk_pw = g.pw;
+    plan->gather = checked_gather(g, plan->gather, tt);
     plan->workspace -= plan->pad_bytes;
     plan->pad_bytes = 0;
     return 0;
@@ -2405,13 +2487,15 @@ static void shared_pad_extent(const Spkv2Context *ctx, const Spkv2NodeRecord *no
 // written), and this conv skips its padding pass.  The producer still writes
 // the unpadded tensor when anything else reads it.  Packages with a
 // protection plan keep every tensor as written by the reference.
-static int setup_pad_handoff(Spkv2Context *ctx, const Spkv2NodeRecord *node, ConvPlan *plan) {
-    if (!plan->padded || ctx->protection_count > 0) return 0;
+static PadSource pad_source(const Spkv2Context *ctx, const Spkv2NodeRecord *node, const ConvGeom &g) {
+    PadSource src;
+    int Hp = 0, Wp = 0;
+    if (!padded_extent(g, &Hp, &Wp) || ctx->protection_count > 0) return src;
     if (const char *e = getenv("SPKV2_PAD_HANDOFF"))
-        if (e[0] == '0') return 0;
+        if (e[0] == '0') return src;
     const uint32_t t = node->inputs[0];
     const Spkv2NodeRecord *prod = nullptr;
-    int readers = 0;
+    int &readers = src.readers;
     for (uint32_t i = 0; i < ctx->header.num_nodes; i++) {
         const Spkv2NodeRecord *n = &ctx->node_records[i];
         for (uint16_t k = 0; k < n->input_count; k++)
@@ -2422,13 +2506,13 @@ static int setup_pad_handoff(Spkv2Context *ctx, const Spkv2NodeRecord *node, Con
     }
     // through a channel Split (a C2f block's halves): the conv whose output
     // the Split cuts hands over the channel range of this conv's input
-    int m0 = 0;
-    bool via_split = false;
+    int &m0 = src.m0;
+    bool &via_split = src.via_split;
     if (prod && prod->op_type == SPKV2_OP_SPLIT && prod->input_count >= 1 && builtin_runs(ctx, prod->id)) {
         Spkv2AttrRecord attr;
         const Spkv2TensorRecord *sr = rec(ctx, prod->inputs[0]);
         if (spkv2_ctx_get_attr(ctx, prod, &attr) != 0 || sr->rank != 4 || (attr.axis < 0 ? attr.axis + 4 : attr.axis) != 1)
-            return 0;
+            return src;
         for (uint16_t k = 0; k < prod->output_count && prod->outputs[k] != t; k++) m0 += rec(ctx, prod->outputs[k])->shape[1];
         const uint32_t s_in = prod->inputs[0];
         const Spkv2NodeRecord *sp = prod;
@@ -2440,26 +2524,33 @@ static int setup_pad_handoff(Spkv2Context *ctx, const Spkv2NodeRecord *node, Con
         }
         via_split = true;
     }
-    if (!prod || prod->op_type != SPKV2_OP_CONV || prod->output_count != 1) return 0;
-    if (!builtin_runs(ctx, prod->id) || !builtin_runs(ctx, node->id)) return 0;  // a user kernel runs one end
-    if (ctx->plan_dtors[prod->id] != conv_plan_free) return 0;
+    if (!prod || prod->op_type != SPKV2_OP_CONV || prod->output_count != 1) return src;
+    if (!builtin_runs(ctx, prod->id) || !builtin_runs(ctx, node->id)) return src;  // a user kernel runs one end
+    if (ctx->plan_dtors[prod->id] != conv_plan_free) return src;
     ConvPlan *pp = static_cast<ConvPlan *>(ctx->plans[prod->id]);
-    if (!pp || (pp->path != CONV_IGEMM_F32 && pp->path != CONV_SMALLK_F32)) return 0;
-    const ConvGeom &g = plan->g;
-    if (pp->g.N != g.N || pp->g.OH != g.H || pp->g.OW != g.W) return 0;
-    if (via_split ? m0 + g.C > pp->g.M : pp->g.M != g.C) return 0;
+    if (!pp || (pp->path != CONV_IGEMM_F32 && pp->path != CONV_SMALLK_F32)) return src;
+    if (pp->g.N != g.N || pp->g.OH != g.H || pp->g.OW != g.W) return src;
+    if (via_split ? m0 + g.C > pp->g.M : pp->g.M != g.C) return src;
+    src.producer = pp;
+    return src;
+}
+
+static int setup_pad_handoff(const Spkv2Context *ctx, const Spkv2NodeRecord *node, ConvPlan *plan, const PadSource &src) {
+    ConvPlan *pp = src.producer;
+    if (!plan->padded || !pp) return 0;
     if (pp->pad_out) {
         // the producer already hands this tensor to an earlier consumer: a
         // consumer with the same padded geometry and channel range reads
         // that consumer's buffer (the producer writes y as well, since the
         // tensor has more than one reader)
-        if (pp->pad_Hp == plan->Hp && pp->pad_Wp == plan->Wp && pp->pad_pt == plan->pt && pp->pad_pl == plan->pl &&
-            pp->pad_m0 == m0 && pp->pad_C == (via_split ? g.C : 0)) {
+        if (shares_pad(src, plan)) {
             plan->pad_in = pp->pad_out;
             plan->pad_in_shared = true;
         }
         return 0;
     }
+    const ConvGeom &g = plan->g;
+    const uint32_t t = node->inputs[0];
     bool is_output = false;
     for (size_t i = 0; i < ctx->output_count; i++)
         if (ctx->output_ids[i] == t) is_output = true;
@@ -2472,9 +2563,9 @@ static int setup_pad_handoff(Spkv2Context *ctx, const Spkv2NodeRecord *node, Con
     pp->pad_Wp = plan->Wp;
     pp->pad_pt = plan->pt;
     pp->pad_pl = plan->pl;
-    pp->pad_m0 = m0;
-    pp->pad_C = via_split ? g.C : 0;
-    pp->y_needed = via_split || readers > 1 || is_output;  // through a Split: the Split reads all of it
+    pp->pad_m0 = src.m0;
+    pp->pad_C = src.via_split ? g.C : 0;
+    pp->y_needed = src.via_split || src.readers > 1 || is_output;  // through a Split: the Split reads all of it
     return 0;
 }
 
@@ -2685,8 +2776,9 @@ int conv_prepare(Spkv2Context *ctx, const Spkv2NodeRecord *node, size_t *ws) {
         } else {
             int hp = 0, wp = 0;
             shared_pad_extent(ctx, node, g, &hp, &wp);
-            rc = plan_igemm_f32(ctx->stream, g, w, plan, hp, wp);
-            if (rc == 0) rc = setup_pad_handoff(ctx, node, plan);
+            const PadSource src = pad_source(ctx, node, g);
+            rc = plan_igemm_f32(ctx->stream, g, w, plan, hp, wp, src);
+            if (rc == 0) rc = setup_pad_handoff(ctx, node, plan, src);
             if (rc == 0) rc = use_implicit_padding(plan);
             if (rc == 0) set_kernel_name(ctx, node, igemm_name(plan) + (plan->pad_in ? "+handoff" : ""));
         }

@@ -13,6 +13,8 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+from .helpers import rng_inputs
+
 pytestmark = pytest.mark.gpu
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -169,8 +171,6 @@ def test_tuner_times_ordinary_operands(gpu, monkeypatch, capfd):
     """The tuner's time of its choice is that of ordinary values (at which
     the chip lowers its clock: 20% here), not that of zeros, which is below
     the layer's node time on zeros by what the node's events take."""
-    import numpy as np
-
     from spinnv2_amd.runtime import Model
     from spinnv2_amd.spk import models, write_spk
 
@@ -198,3 +198,51 @@ def test_tuner_times_ordinary_operands(gpu, monkeypatch, capfd):
     tuned = [line for line in capfd.readouterr().err.splitlines() if line.startswith("[tune]   ")]
     best = float(tuned[0].split()[-1])
     assert best > took["zeros"], (best, took)
+
+
+def test_tuner_times_the_padding_that_runs(gpu, monkeypatch, capfd):
+    """A padded layer that pads its own input is tuned with its copy or its
+    checked taps, as it runs then; one whose input another layer hands over
+    padded is tuned on padded planes."""
+    from spinnv2_amd.runtime import Model
+    from spinnv2_amd.spk import models, write_spk
+    from spinnv2_amd.spk.graph import Graph
+
+    for k in ("SPKV2_TUNE_DB", "SPKV2_CONV_CFG", "SPKV2_CONV_SPLITK", "SPKV2_CONV_HYBRID", "SPKV2_CONV_TUNE",
+              "SPKV2_IMPLICIT_PAD"):
+        monkeypatch.delenv(k, raising=False)
+    monkeypatch.setenv("SPKV2_TUNE_LOG", "1")
+    monkeypatch.setenv("SPKV2_TUNE_TIE", "0")  # the fastest candidate, first in the log
+
+    def tuned(g):
+        """Per layer the log's candidates, and the kernel that runs."""
+        capfd.readouterr()
+        with Model(write_spk(g, "mi355x")) as mdl:
+            mdl(*rng_inputs(g))
+            names = [mdl.kernel_name(i) for i in range(len(g.nodes))]
+        layers = []
+        for line in capfd.readouterr().err.splitlines():
+            if line.startswith("[tune] conv"):
+                layers.append([])
+            elif line.startswith("[tune]   ") and layers:
+                layers[-1].append(line)
+        return layers, names
+
+    forms = set()
+    for n, c, h, w, m, s in [(4, 40, 23, 19, 72, 1), (6, 104, 35, 27, 72, 2), (2, 10, 61, 53, 40, 1)]:
+        (lines,), (name,) = tuned(models.single_conv(n, c, h, w, m, 3, s, 1))
+        for line in lines:
+            assert (",copy" in line) != (",ipad" in line), line
+            forms.add(",ipad" if ",ipad" in line else ",copy")
+        assert (",ipad" in lines[0]) == (",ipad" in name), (lines[0], name)
+    assert len(forms) == 2, forms
+
+    g = Graph("two")
+    rng = np.random.default_rng(5)
+    y = g.input("x", [3, 40, 21, 19])
+    for k, pad in ((1, 0), (3, 1)):
+        y = g.conv(y, rng.standard_normal((40, 40, k, k)).astype(np.float32), np.zeros(40, np.float32), pad=pad)
+    g.mark_output(y)
+    layers, names = tuned(g)
+    assert "+handoff" in names[1], names
+    assert len(layers) == 2 and not any(",copy" in line or ",ipad" in line for lines in layers for line in lines)
