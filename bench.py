@@ -2,7 +2,7 @@
 
 A step is one spkv2_run of the whole network over one batch whose input is
 already resident in HBM (a device buffer bound with spkv2_bind_input).
-Workload (BASELINE.json configs[2]): ResNet-101-style bottleneck CNN, batch
+Workload: ResNet-101-style bottleneck CNN, batch
 64, He-normal weights with BN folded, N(0,1) input, seed 42 (synthetic data,
 random-init weights of the real architecture).
 
@@ -13,9 +13,13 @@ Reported:
   roofline       conv implicit-GEMM throughput: conv FLOP per step / the
                  summed kernel-trace durations of the conv nodes' launches
                  per step (the committed rocprofv3 summary of this workload),
-                 against the fp32 MFMA peak; beside it the live figures of
-                 this run: HIP events around every node on the run stream in
-                 a separate eager pass of W + K steps, and the timed step;
+                 against the peak of the units that run them (`peak`: the convs
+                 on bf16 parts at a sixth of the dense bf16 rate, six products
+                 each, the others at the fp32 MFMA rate, weighted by FLOP);
+                 `fp32_mfma_frac` is the metric's share of the fp32 MFMA peak;
+                 beside it the live figures of this run: HIP events around
+                 every node on the run stream in a separate eager pass of W + K
+                 steps, and the timed step;
   graph_matches_eager  the timed graph replay's output is bit-identical to
                  the eager pass's output of the same input;
   b1_*           batch-1 latency and images/sec (HIP-graph replay);
@@ -23,7 +27,7 @@ Reported:
                  x86) on one batch-1 image, timed on the host;
   int8, elementwise, yolo   INT8 ResNet-50, the memory-bound ops against
                  the HBM peak, YOLOv10n 640 images/s (sections of their own);
-  int8_config_mode  INT8 ResNet-50 in BASELINE configs[4]'s own semantics
+  int8_config_mode  INT8 ResNet-50 in the INT8 configuration's semantics
                  (asymmetric activations, int8 tensors between nodes,
                  fixed-point requantization), against the int8 MFMA peak.
 
@@ -46,6 +50,8 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 FP32_MFMA_PEAK_TFLOPS = 157.3
+BF16_MFMA_PEAK_TFLOPS = 2500.0
+PARTS_PEAK_TFLOPS = BF16_MFMA_PEAK_TFLOPS / 6  # a product of floats is six products of bf16 parts
 INT8_MFMA_PEAK_TOPS = 5000.0
 HBM_PEAK_GBPS = 8000.0
 
@@ -248,7 +254,7 @@ def batch1_latency(depth: int, steps: int, lib, eager: bool = False) -> tuple[fl
 
 def int8_resnet50(lib, steps: int, warmup: int, b1_steps: int, batch: int = 64, node_report: bool = False,
                   eager: bool = False) -> dict:
-    """INT8 ResNet-50 (BASELINE configs[4]): per-channel symmetric int8
+    """INT8 ResNet-50: per-channel symmetric int8
     weights, per-tensor activation scales calibrated on 16 seeded single-image
     batches with the repo's fp32 forward, int32 accumulation, reference
     dequantization.  Returns images/s at `batch`, batch-1 latency, and the
@@ -391,7 +397,7 @@ def int8_resnet50(lib, steps: int, warmup: int, b1_steps: int, batch: int = 64, 
 
 def int8_config_mode(lib, steps: int, warmup: int, b1_steps: int, batch: int = 64, node_report: bool = False,
                      eager: bool = False) -> dict:
-    """INT8 ResNet-50 224x224 in BASELINE configs[4]'s own semantics (no
+    """INT8 ResNet-50 224x224 in the INT8 configuration's semantics (no
     reference counterpart): per-channel symmetric int8 weights, per-tensor
     asymmetric activation scales and zero points from min/max over 16
     seeded calibration batches, int8 tensors between nodes, int32
@@ -469,7 +475,7 @@ def int8_config_mode(lib, steps: int, warmup: int, b1_steps: int, batch: int = 6
     out = {"workload": "resnet50_int8_config_224", "batch": batch, "images_per_sec": batch * steps / elapsed,
            "ms_per_step": elapsed * 1e3 / steps, "timed_mode": "eager" if eager else "hip_graph",
            "graph_matches_eager": graph_same,
-           "semantics": "BASELINE configs[4]: per-channel symmetric int8 weights, per-tensor asymmetric int8 "
+           "semantics": "INT8 configuration: per-channel symmetric int8 weights, per-tensor asymmetric int8 "
                         "activations (min/max over 16 calibration batches), int8 tensors between nodes, int32 "
                         "accumulate, fixed-point requantize (round half away), fused Relu clamp; no reference "
                         "counterpart (checked against the oracle's restatement)",
@@ -509,7 +515,7 @@ def int8_config_mode(lib, steps: int, warmup: int, b1_steps: int, batch: int = 6
 
 
 def yolo_v10n(lib, steps: int, node_report: bool = False, eager: bool = False, batches=(1, 16)) -> dict:
-    """YOLOv10n-style detector (BASELINE configs[3]) at 640x640, batch 1 and
+    """YOLOv10n-style detector at 640x640, batch 1 and
     16: images/s from HIP-graph replays of the node loop (the whole YOLO op
     set on the device: C2f Split/Concat, SPPF, PSA MatMul + Softmax, Resize,
     DFL Softmax, TopK, GatherElements), plus the node time by op type from an
@@ -613,7 +619,7 @@ def main() -> None:
     ap.add_argument("--no-int8", action="store_true", help="skip the INT8 ResNet-50 section")
     ap.add_argument("--int8-only", action="store_true", help="run only the INT8 ResNet-50 section")
     ap.add_argument("--int8-config-only", action="store_true",
-                    help="run only the INT8 ResNet-50 section in BASELINE configs[4]'s own semantics")
+                    help="run only the INT8 ResNet-50 section in the INT8 configuration's semantics")
     ap.add_argument("--no-int8-config", action="store_true", help="skip the INT8 configuration-semantics section")
     ap.add_argument("--no-elementwise", action="store_true", help="skip the memory-bound op section")
     ap.add_argument("--no-yolo", action="store_true", help="skip the YOLOv10n section")
@@ -744,6 +750,10 @@ def main() -> None:
             if nid in flops_per_node:
                 extra = f" {flops_per_node[nid] / ms / 1e9:.1f} TFLOP/s"
             log(f"node {nid:3d} {n.op_type:18s} {m.kernel_name(nid):44s} {ms:8.3f} ms{extra}")
+    # the convs' peak: the time their FLOP take at the rate of the unit each runs on
+    on_parts = [nid for nid in flops_per_node if "conv_split_f32" in m.kernel_name(nid)]
+    parts_flops = sum(flops_per_node[nid] for nid in on_parts)
+    conv_peak = conv_flops / (parts_flops / PARTS_PEAK_TFLOPS + (conv_flops - parts_flops) / FP32_MFMA_PEAK_TFLOPS)
     m.close()
     xin.free()
     ms_per_step = elapsed * 1e3 / args.steps
@@ -794,18 +804,22 @@ def main() -> None:
         "node_ms_per_step": total_node_ms,
         "graph_matches_eager": graph_same,
         "b1_graph_matches_eager": b1_same,
-        "roofline": {"bound": "mfma", "achieved": roof_tflops, "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": roof_tflops / FP32_MFMA_PEAK_TFLOPS,
+        "roofline": {"bound": "mfma", "achieved": roof_tflops, "peak": conv_peak, "unit": "TFLOP/s",
+                     "frac": roof_tflops / conv_peak,
+                     "peak_basis": f"{len(on_parts)} of {len(conv_nodes)} convs ({parts_flops / conv_flops:.3f} of the "
+                                   f"FLOP) on bf16 parts at {PARTS_PEAK_TFLOPS:.1f} TFLOP/s (dense bf16 / 6), the rest "
+                                   f"at the fp32 MFMA peak of {FP32_MFMA_PEAK_TFLOPS}",
+                     "fp32_mfma_frac": roof_tflops / FP32_MFMA_PEAK_TFLOPS,
                      "basis": ("summed kernel-trace durations of the conv nodes' launches per step "
                                "(profiles/conv_igemm_f32_resnet101_b64_kernel_stats.txt, result conv_kernels_ms_per_run)"
                                if trace_ms else "HIP events around every conv node (no committed trace for this shape)"),
                      "kernel_ms_per_step": trace_ms,
                      "event_basis": {"conv_ms_per_step": conv_ms, "tflops": conv_tflops,
-                                     "frac": conv_tflops / FP32_MFMA_PEAK_TFLOPS,
+                                     "frac": conv_tflops / conv_peak,
                                      "note": "HIP events per node, eager pass of this run: an upper bound of the time"},
                      "step_basis": {"ms_per_step": ms_per_step,
                                     "tflops": conv_flops / (ms_per_step * 1e-3) / 1e12,
-                                    "frac": conv_flops / (ms_per_step * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
+                                    "frac": conv_flops / (ms_per_step * 1e-3) / 1e12 / conv_peak,
                                     "note": "conv FLOP over the whole timed graph step (all kernels)"},
                      "traffic": traffic.get("conv_hbm_bytes_per_step") if traffic else None,
                      "traffic_basis": "HBM bytes of all conv launches of one step (rocprofv3 FETCH_SIZE + "
