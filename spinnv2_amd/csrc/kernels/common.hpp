@@ -49,6 +49,11 @@ inline void div_magic(unsigned d, unsigned *m, int *s) {
     *m = static_cast<unsigned>(((uint64_t(1) << *s) + d - 1) / d);
 }
 
+// Byte offset of a buffer access, with no scalar offset beside it, that is to
+// do nothing: past the end of every tensor (they are below 2 GiB), and no
+// offset into a tensor that is added to it wraps.
+constexpr int kPastTensor = -0x7fffffff - 1;
+
 inline size_t elem_count(const Spkv2TensorRecord *r) {
     size_t n = 1;
     for (uint16_t i = 0; i < r->rank; i++) n *= r->shape[i];

@@ -779,8 +779,8 @@ __global__ void __launch_bounds__(256) conv_thin_f32(IgemmArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int n = n0 + 16 * j + l16;
-        obase[j] = kOobOffset;
-        pbase[j] = kOobOffset;
+        obase[j] = kPastTensor;
+        pbase[j] = kPastTensor;
         if (n < a.Ntot) {
             const int img = n / a.OHW;
             const int sp = n - img * a.OHW;
@@ -818,7 +818,7 @@ __global__ void __launch_bounds__(256) conv_thin_f32(IgemmArgs a) {
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                     rv[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                          rrs, m0 + r < a.M ? obase[j] + (m0 + r) * ohw4 : kOobOffset, 0, 0));
+                                                          rrs, m0 + r < a.M ? obase[j] + (m0 + r) * ohw4 : kPastTensor, 0, 0));
                 v += rv;
             }
 #pragma unroll
@@ -829,14 +829,14 @@ __global__ void __launch_bounds__(256) conv_thin_f32(IgemmArgs a) {
                     const unsigned mc = static_cast<unsigned>(m0 + r - a.yp_m0);
                     __builtin_amdgcn_raw_buffer_store_b32(
                         __float_as_uint(v[r]), prs,
-                        mc < static_cast<unsigned>(a.yp_C) ? pbase[j] + static_cast<int>(mc) * plane4 : kOobOffset, 0, 0);
+                        mc < static_cast<unsigned>(a.yp_C) ? pbase[j] + static_cast<int>(mc) * plane4 : kPastTensor, 0, 0);
                 }
             }
             if (a.y) {
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), yrs,
-                                                          m0 + r < a.M ? obase[j] + (m0 + r) * a.y_cstride * 4 : kOobOffset,
+                                                          m0 + r < a.M ? obase[j] + (m0 + r) * a.y_cstride * 4 : kPastTensor,
                                                           0, 0);
             }
         }
@@ -1084,7 +1084,7 @@ __global__ void __launch_bounds__(256) conv_smallk_f32(SmallkArgs a) {
                             static_cast<unsigned>(ihb + (dd >> 16)) < static_cast<unsigned>(a.H) &&
                             static_cast<unsigned>(iwb + (dd & 0xffff)) < static_cast<unsigned>(a.W);
             xv[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                  xrs, ok ? (base + toff[k]) * 4 : kOobOffset, 0, 0));
+                                                  xrs, ok ? (base + toff[k]) * 4 : kPastTensor, 0, 0));
             okm |= static_cast<unsigned>(ok) << j;
         }
 #pragma unroll

@@ -493,7 +493,7 @@ __device__ __forceinline__ void i8_epilogue(intx16 (&acc)[TM][TN], const I8Args 
         const int sp = n - img * a.OHW;
         obase[j] = n < a.Ntot
                        ? (static_cast<unsigned>(img) * M * static_cast<unsigned>(a.OHW) + static_cast<unsigned>(sp)) * 4u
-                       : static_cast<unsigned>(kOob);
+                       : static_cast<unsigned>(kPastTensor);
     }
     if (a.mode == 2) {
         const __amdgpu_buffer_rsrc_t wrs =
@@ -505,7 +505,7 @@ __device__ __forceinline__ void i8_epilogue(intx16 (&acc)[TM][TN], const I8Args 
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const unsigned m = mrow[i] + 8 * (r >> 2) + (r & 3);
-                    __builtin_amdgcn_raw_buffer_store_b32(acc[i][j][r], wrs, m < M ? obase[j] + m * ohw4 : kOob, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b32(acc[i][j][r], wrs, m < M ? obase[j] + m * ohw4 : kPastTensor, 0, 0);
                 }
         return;
     }
@@ -556,7 +556,7 @@ __device__ __forceinline__ void i8_epilogue(intx16 (&acc)[TM][TN], const I8Args 
                 for (int r = 0; r < 16; r++) {
                     const unsigned m = mrow[i] + 8 * (r >> 2) + (r & 3);
                     rv[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                          rrs, m < M ? obase[j] + m * ohw4 : kOob, 0, 0));
+                                                          rrs, m < M ? obase[j] + m * ohw4 : kPastTensor, 0, 0));
                 }
                 v += rv;
             }
@@ -606,7 +606,7 @@ __device__ __forceinline__ void i8_epilogue(intx16 (&acc)[TM][TN], const I8Args 
                     const unsigned m = mrow[i] + 8 * (r >> 2) + (r & 3);
                     // __float_as_uint takes the element by value
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), yrs,
-                                                          m < M ? obase[j] + m * ohw4 : kOob, 0, 0);
+                                                          m < M ? obase[j] + m * ohw4 : kPastTensor, 0, 0);
                 }
             }
         }

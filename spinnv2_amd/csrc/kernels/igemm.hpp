@@ -9,8 +9,8 @@ namespace spk::kern {
 // gfx9 buffer resource word 3 (raw, untyped loads); loads whose offset is at
 // or beyond num_records return 0.
 constexpr int kBufferWord3 = 0x00020000;
-// byte offset that is out of range for every tensor (they are < 2 GiB), and
-// still does not wrap when a valid offset is added to it
+// byte offset that is out of range for every B source (they are shorter:
+// plan_igemm_f32), and still does not wrap when a valid offset is added to it
 constexpr int kOobOffset = 0x7fff0000;
 
 // Tiles of out-of-range entries that a k -> offset table (and a tap table) has
@@ -73,11 +73,11 @@ __device__ __forceinline__ void store_rows(const Block &v, int r, __amdgpu_buffe
     if (quads) {
         const uintx4 o = {__float_as_uint(v[r]), __float_as_uint(v[r + 1]), __float_as_uint(v[r + 2]),
                           __float_as_uint(v[r + 3])};
-        __builtin_amdgcn_raw_buffer_store_b128(o, rs, left > 0 ? off : kOobOffset, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(o, rs, left > 0 ? off : kPastTensor, 0, 0);
     } else {
 #pragma unroll
         for (int e = 0; e < 4; e++)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r + e]), rs, e < left ? off + 4 * e : kOobOffset, 0,
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r + e]), rs, e < left ? off + 4 * e : kPastTensor, 0,
                                                   0);
     }
 }
@@ -113,7 +113,7 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             const int n = nt * BN + (wn * TN + j) * BS + row;
-            obase[j] = n >= a.Ntot ? kOobOffset
+            obase[j] = n >= a.Ntot ? kPastTensor
                        : ROWS      ? (slice * a.ws_ld + n - a.ws_n0) * a.M * 4
                                    : (slice * a.M * a.ws_ld + n - a.ws_n0) * 4;
         }
@@ -137,7 +137,7 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
                     const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
-                    const int off = m < a.M ? obase[j] + m * a.ws_ld * 4 : kOobOffset;
+                    const int off = m < a.M ? obase[j] + m * a.ws_ld * 4 : kPastTensor;
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][r]), wrs, off, 0, 0);
                 }
         return;  // splitk_epilogue sums the partials
@@ -153,8 +153,8 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
         const int sp = n - img * a.OHW;
         const int oh = sp / a.OW;
         const int ow = sp - oh * a.OW;
-        obase[j] = n < a.Ntot ? (img * a.y_img_stride + sp) * 4 : kOobOffset;
-        pbase[j] = n < a.Ntot ? (img * a.yp_C * a.yp_plane + (oh + a.yp_pt) * a.yp_Wp + ow + a.yp_pl) * 4 : kOobOffset;
+        obase[j] = n < a.Ntot ? (img * a.y_img_stride + sp) * 4 : kPastTensor;
+        pbase[j] = n < a.Ntot ? (img * a.yp_C * a.yp_plane + (oh + a.yp_pt) * a.yp_Wp + ow + a.yp_pl) * 4 : kPastTensor;
     }
     float *const any = a.y ? a.y : a.yp;
     const __amdgpu_buffer_rsrc_t yrs =
@@ -196,7 +196,7 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
                             const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
                             v[j][r] += __builtin_bit_cast(
                                 float, __builtin_amdgcn_raw_buffer_load_b32(
-                                           rrs, m < a.M ? obase[j0 + j] + m * 4 : kOobOffset, 0, 0));
+                                           rrs, m < a.M ? obase[j0 + j] + m * 4 : kPastTensor, 0, 0));
                         }
                 }
 #pragma unroll
@@ -220,7 +220,7 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
                         const int m = mrow[i] + 8 * (r >> 2) + (r & 3);
                         rv[j][r] = __builtin_bit_cast(
                             float, __builtin_amdgcn_raw_buffer_load_b32(
-                                       rrs, m < a.M ? obase[j0 + j] + m * ohw4 : kOobOffset, 0, 0));
+                                       rrs, m < a.M ? obase[j0 + j] + m * ohw4 : kPastTensor, 0, 0));
                     }
 #pragma unroll
                 for (int j = 0; j < JG; j++) v[j] += rv[j];
@@ -244,7 +244,7 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
                         __builtin_amdgcn_raw_buffer_store_b32(
                             __float_as_uint(v[j][r]), prs,
                             mc < static_cast<unsigned>(a.yp_C) ? pbase[j0 + j] + static_cast<int>(mc) * plane4
-                                                               : kOobOffset,
+                                                               : kPastTensor,
                             0, 0);
                     }
             }
@@ -257,7 +257,7 @@ __device__ __forceinline__ void igemm_epilogue(const IgemmArgs &a, const Block (
                         // __float_as_uint takes the element by value (a bit
                         // cast applied to a vector element reads element 0)
                         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j][r]), yrs,
-                                                              m < a.M ? obase[j0 + j] + m * ycs4 : kOobOffset, 0, 0);
+                                                              m < a.M ? obase[j0 + j] + m * ycs4 : kPastTensor, 0, 0);
                     }
             }
         }
