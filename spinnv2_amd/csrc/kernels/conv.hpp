@@ -36,6 +36,13 @@ enum ConvPath {
     CONV_Q8 = 5
 };
 
+// Longest buffer that channel-slice views lie in, and the most bytes of rows
+// and columns ahead of a tensor that checked taps may count from (implicit
+// padding): an input's extent, these added, stays below the offset that stands
+// for out of range (igemm.hpp).
+constexpr int64_t kMaxViewBytes = 0x7e000000;
+constexpr int64_t kMaxBytesAhead = 0x01ff0000;
+
 // How an fp32 implicit-GEMM B source is laid out beyond its k-offset table.
 // Per tap, for the skinny kernel: k = c * taps + tap sits at c * cstride +
 // (tap / KW) * tap_h + (tap % KW) * tap_w elements from the column's base (C

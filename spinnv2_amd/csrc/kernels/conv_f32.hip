@@ -1522,6 +1522,7 @@ bool takes_checks(const ConvGeom &g, int cfg, int Hp, int Wp) {
     const TileCfg &t = kCfgs[cfg];
     if (t.skinny_waves > 0 || t.thin_mb > 0) return false;
     if (g.H >= 16384 || g.W >= 16384 || (g.KH - 1) * g.dh >= 32768 || (g.KW - 1) * g.dw >= 32768) return false;
+    if ((static_cast<int64_t>(g.ph) * g.W + g.pw) * 4 > kMaxBytesAhead) return false;
     const char *e = getenv("SPKV2_IMPLICIT_PAD");
     if (e && e[0] == '0') return false;
     const bool parts = t.split_threads > 0;

@@ -10,7 +10,8 @@ namespace spk::kern {
 // or beyond num_records return 0.
 constexpr int kBufferWord3 = 0x00020000;
 // byte offset that is out of range for every B source (they are shorter:
-// plan_igemm_f32), and still does not wrap when a valid offset is added to it
+// plan_igemm_f32, kMaxViewBytes), and still does not wrap when a valid offset is
+// added to it
 constexpr int kOobOffset = 0x7fff0000;
 
 // Tiles of out-of-range entries that a k -> offset table (and a tap table) has

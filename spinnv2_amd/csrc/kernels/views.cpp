@@ -212,7 +212,7 @@ void setup_head_views(Spkv2Context *ctx, const Uses &u) {
             continue;
         const int64_t N = orr->shape[0], C = orr->shape[1], L = orr->shape[2];
         const int64_t zbytes = N * C * L * 4;
-        if (zbytes >= (int64_t(1) << 31)) continue;
+        if (zbytes > kMaxViewBytes) continue;
         struct Place {
             uint32_t t;
             int64_t off;  // elements from the buffer's start
@@ -398,7 +398,7 @@ int setup_concat_views(Spkv2Context *ctx) {
         const Spkv2TensorRecord *yr = rec(ctx, o);
         const int64_t N = yr->shape[0], CZ = yr->shape[1], HW = static_cast<int64_t>(yr->shape[2]) * yr->shape[3];
         const int64_t zbytes = N * CZ * HW * 4;
-        if (zbytes >= (int64_t(1) << 31)) continue;  // 32-bit byte offsets in the kernels
+        if (zbytes > kMaxViewBytes) continue;  // 32-bit byte offsets in the kernels
         bool shapes = true;
         std::vector<int64_t> c(k->input_count + 1, 0);
         for (uint16_t i = 0; i < k->input_count; i++) {
