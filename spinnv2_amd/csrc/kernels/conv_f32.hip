@@ -1436,7 +1436,7 @@ double model_us(int c, const TileCounts &tc, int M, int Ntot) {
 // split-K cuts k (slices of kt_per_split * BK k, summed in slice order by the
 // epilogue) and, for the hybrid schedule, on which columns are cut (ws_n0).
 // The skinny and thin kernels sum in orders of their own (tap-major k, wave
-// partials through LDS).
+// partials through LDS), and the tiles on bf16 parts share one of theirs.
 std::string numerics_class(int c, const TileCounts &tc) {
     const TileCfg &t = kCfgs[c];
     if (t.skinny_waves > 0) return "skinny" + std::to_string(t.skinny_waves);

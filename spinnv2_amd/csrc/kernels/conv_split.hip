@@ -7,7 +7,10 @@
 // runs 16 times as many operations a cycle as v_mfma_f32_32x32x2_f32: 2.7
 // times the fp32 rate at the clocks' limit, though at this load the chip
 // holds the matrix cores to about 1.5 PFLOP/s, 1.6 times what the fp32 ones
-// reach.  The three products left out are below 2^-25 of the whole each.
+// reach.  The three products left out are below 2^-24 of the whole together
+// (2^-25, 2^-25 and 2^-34).  The split and the six products are those of Henry,
+// Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype
+// For Higher-Precision Computations" (ARITH 2019).
 //
 // Precision: against 64-bit sums of N(0, 1) data the relative error is 5e-8
 // at K = 64, 8.5e-8 at 256 and 2.9e-7 at 2304, where the fp32 MFMA's is

@@ -5,7 +5,7 @@ Each builder emits the ONNX-level graph (Conv, BatchNormalization, Relu, Add,
 pipeline, so the packaged graph is what the reference compiler would produce
 from the same model (BN folded, Conv+Relu, Add+Relu, Conv+Add).
 
-Distributions (BASELINE.json configs): conv / fc weights He-normal
+Distributions: conv / fc weights He-normal
 N(0, sqrt(2 / fan_in)); biases N(0, 0.01); BN gamma ~ U(0.5, 1.5),
 beta, mean ~ N(0, 0.1), var ~ U(0.5, 1.5), eps 1e-5.
 """
@@ -314,7 +314,7 @@ def _psa(g: Graph, p: Params, x: int, c: int) -> int:
 
 def yolo_v10n(batch: int = 1, image: int = 640, seed: int = DEFAULT_SEED, classes: int = 80,
               topk: int = 300) -> Graph:
-    """YOLOv10n-style detector (BASELINE configs[3]): CSP backbone of 3x3/2
+    """YOLOv10n-style detector: CSP backbone of 3x3/2
     Conv+BN+SiLU downsamples 16->32->64->128->256 with C2f split/concat
     blocks, SPPF, a PSA attention block (2 heads over the stride-32 map:
     batched MatMul, Softmax), PAN neck (nearest Resize x2 + Concat), decoupled heads at

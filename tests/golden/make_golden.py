@@ -9,11 +9,11 @@ profiles whose conv kinds its optimized x86 kernels run -- and stores, per
 case, the builder call, the profile, the inputs and the reference runtime's
 output.  The fixtures are data only: the
 tests re-create each package with the same builder call and compare the CPU
-oracle (and, on the GPU box, the MI355X runtime) against the stored output.
+oracle (and, on a GPU, the MI355X runtime) against the stored output.
 
     python tests/golden/make_golden.py          # rewrites tests/golden/*.npz
 
-Needs /root/reference; the GPU box never runs this.
+Needs /root/reference; no GPU test runs this.
 """
 
 from __future__ import annotations
@@ -155,13 +155,13 @@ _MATMUL = [
 for i, kw in enumerate(_MATMUL):
     CASES.append((f"matmul{i}", "matmul_op", kw, "normal"))
 
-# End to end: the LeNet config (BASELINE configs[0]) on U[0,1) input, and a
+# End to end: the LeNet config on U[0,1) input, and a
 # ResNet-18 at 32x32 (every ResNet node kind: stem, pools, basic blocks with
 # projections, ReduceMean, Gemm).
 CASES.append(("lenet", "lenet", {}, "uniform"))
 CASES.append(("resnet18_32px", "resnet", dict(depth=18, batch=2, image=32, classes=10), "normal"))
 CASES.append(("resnet50_32px", "resnet", dict(depth=50, batch=1, image=32, classes=10), "normal"))
-# the YOLOv10n-style detector (BASELINE configs[3]) at 160x160: 525 anchors, TopK(300)
+# the YOLOv10n-style detector at 160x160: 525 anchors, TopK(300)
 CASES.append(("yolov10n_160", "yolo_v10n", dict(image=160), "uniform"))
 
 

@@ -14,7 +14,7 @@ runtime/tests/test_reliability.c scenario.
 
     python tests/golden/reliability/make_reliability.py   # rewrites cases.json, outputs.npz
 
-Needs /root/reference; the GPU box never runs this.
+Needs /root/reference; no GPU test runs this.
 """
 
 from __future__ import annotations

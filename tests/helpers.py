@@ -4,7 +4,7 @@ from __future__ import annotations
 
 import numpy as np
 
-# fp32 max relative error <= 1e-4 per tensor, measured
+# The parity bar: fp32 max relative error <= 1e-4 per tensor, measured
 # tensor-normalized (max|a-b| / max|b|): the reference's own naive and AVX2
 # conv kernels differ by ~1e-4 element-wise on small outputs.
 FP32_TOL = 1e-4

@@ -1,7 +1,7 @@
 """GPU parity on the benchmark configurations at their stated sizes.
 
 ResNet-18 fp32 at 224x224, batch 32, and the INT8 ResNet-50 at 224x224,
-batch 1 and batch 64 (BASELINE configs[1] and [4]), against the CPU oracle
+batch 1 and batch 64, against the CPU oracle
 through the C ABI.  Reference semantics: runtime/kernels/reference/conv/conv.c
 for fp32, runtime/kernels/optimized/conv/conv_int8.c:121-210 for INT8.
 

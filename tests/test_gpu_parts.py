@@ -1,9 +1,9 @@
 """The implicit GEMM on bf16 parts (conv_split.hip) against 64-bit sums.
 
-A float32 operand is the exact sum of three bf16 parts, and the six largest
-of a product's nine part products are summed: the three left out are below
-2^-25 of the product each, and a sum of K products rounds once per 16 of them
-and once per slice, so |error| <= (K / 8 + 16) * 2^-24 * sum |x w| with room
+A float32 operand, scaled by 2^24, is the exact sum of three bf16 parts, and
+the six largest of a product's nine part products are summed: the three left
+out are below 2^-24 of the product together, and a sum of K products rounds
+once per 16 of them and once per slice, so |error| <= (K / 8 + 16) * 2^-24 * sum |x w| with room
 for the matrix core's own order within a step.
 """
 
@@ -276,3 +276,19 @@ def test_parts_implicit_padding(gpu, monkeypatch, case, cfg, implicit):
     assert "conv_split_f32" in name, name
     assert (",ipad" in name) == (implicit == "1" and k <= 15), name
     assert tnorm_err(got, run_oracle(blob, xs)[0]) <= FP32_TOL
+
+
+@pytest.mark.parametrize("split", [1, 2])
+def test_parts_tiles_share_one_summation_order(gpu, monkeypatch, split):
+    """As for the fp32 tiles: timing may choose among the tiles, and between a
+    copy and checked taps, for the same cut of k."""
+    g = models.single_conv(2, 64, 15, 14, 100, 3, 1, 1, act=None)
+    xs = rng_inputs(g)
+    outs = []
+    for cfg in PARTS_CFGS:
+        _force(monkeypatch, cfg, split)
+        for implicit in ("0", "1"):
+            monkeypatch.setenv("SPKV2_IMPLICIT_PAD", implicit)
+            outs.append(run_gpu(write_spk(g, "mi355x"), xs)[0])
+    for y in outs[1:]:
+        np.testing.assert_array_equal(y.view(np.uint32), outs[0].view(np.uint32))

@@ -1,11 +1,11 @@
 """GPU parity of the INT8 configuration with int8 tensors between nodes
-(BASELINE configs[4]: per-channel symmetric int8 weights, per-tensor
+(per-channel symmetric int8 weights, per-tensor
 asymmetric activations from min/max calibration, int32 accumulation,
 fixed-point requantization with round-half-away, fused Relu clamp).
 
 The reference runtime has no such mode, so the checker is the oracle's
 restatement (oracle/spk_oracle.c, oracle_q8_*), pinned on the CPU by
-tests/test_oracle_q8.py.  The bar is the north star's for INT8: the int32
+tests/test_oracle_q8.py.  The bar for INT8: the int32
 accumulators and the requantized int8 outputs bit-exact, here for every
 int8 tensor of the network (read back from the device), and the dequantized
 spatial mean (an exact integer sum and two IEEE double operations) bit-exact.
